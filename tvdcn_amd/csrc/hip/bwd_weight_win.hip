@@ -500,18 +500,23 @@ hipError_t launch_k1(const Geo &g, const WinTiles &wt, const WeightWin &ww, cons
     return hipGetLastError();
 }
 
-// the fp32 instantiation, and (with an operand flag) the 16-bit one beside it
+// fp32: the fp32 loop, and (with an operand flag) the 16-bit one beside it. fp16 / bf16 operands are the
+// 16-bit loop's own and never flagged: that launch alone (the unselected one cost 4.5 us a call)
 template <int DIM, typename T, bool FULL, int MB, int TG, int TMV, int KPV>
 hipError_t launch_k(const Geo &g, const WinTiles &wt, const WinTiles &wt16, const WeightWin &ww, const void *z,
                     const void *xcl, const void *offset, const void *mask, void *part, const int *flag,
                     const void *zw, hipStream_t s) {
     if (wt.tpp > TMV || wt16.tpp != wt.tpp) return hipErrorInvalidValue;   // a pass must fit the tap slots
-    if (flag != nullptr) {
-        const hipError_t e = launch_k1<DIM, T, FULL, MB, TG, TMV, KPV, true>(g, wt16, ww, z, xcl, offset, mask, part,
-                                                                              flag, zw, s);
-        if (e != hipSuccess) return e;
+    if constexpr (npiece_of<T>() == 1) {
+        return launch_k1<DIM, T, FULL, MB, TG, TMV, KPV, true>(g, wt16, ww, z, xcl, offset, mask, part, nullptr, zw, s);
+    } else {
+        if (flag != nullptr) {
+            const hipError_t e = launch_k1<DIM, T, FULL, MB, TG, TMV, KPV, true>(g, wt16, ww, z, xcl, offset, mask,
+                                                                                  part, flag, zw, s);
+            if (e != hipSuccess) return e;
+        }
+        return launch_k1<DIM, T, FULL, MB, TG, TMV, KPV, false>(g, wt, ww, z, xcl, offset, mask, part, flag, nullptr, s);
     }
-    return launch_k1<DIM, T, FULL, MB, TG, TMV, KPV, false>(g, wt, ww, z, xcl, offset, mask, part, flag, nullptr, s);
 }
 
 template <typename T>
