@@ -10,10 +10,15 @@
 // compute_grad_mask per batch block (tvdcn/csrc/ops/cuda/deform_conv2d_kernel.cpp:518-598,
 // kernels deform_conv2d_common_kernels.cu:258-624, and the 1D/3D twins).
 //
-// Workgroup = one tile: a box of 256 column pixels of one image (16x16 in 2D,
-// 256 in 1D, 4x8x8 in 3D) x 16 sampled-side channels x every tap; eight waves
-// (two per SIMD, so one wave's loads overlap the other's MFMAs), each owning 32
-// pixels; one workgroup per CU (the window takes most of the 160 KB of LDS).
+// Workgroup = one pass of up to nine taps of one tile: a box of 256 column pixels of one image
+// (16x16 in 2D, 256 in 1D, 4x8x8 in 3D) x 16 sampled-side channels; one workgroup per CU (the
+// window takes most of the 160 KB of LDS). The passes of a tile are workgroups of their own: a
+// loop over them had the compiler hoist the per-tile values of every phase above it (240-256
+// registers and ~150 spilled scalars per kernel, now 105-176 and 5-60: one-pass layers -2% of
+// their training step from that alone), and the passes of a small grid run side by side. Sixteen
+// waves of 16 pixels (four per SIMD), or eight of 32 pixels where the K loop counts (see
+// plan_data_win): the 3D epilogue, which waits on LDS and memory, ran 1.63 -> 1.48 ms at 27 taps,
+// 64 channels, 2 x 16x56x56 with sixteen.
 //   * K loop over the GEMM-side channels m, operands straight from global memory
 //     into registers (the next step's prefetched while the MFMAs of the current one
 //     run): wave w computes Gt[c][px] for its 32 pixels, so each lane holds four
@@ -35,26 +40,23 @@
 //     integer LDS atomics (ds_add_u32 measured at ~5 cycles per wave instruction
 //     on gfx950, ds_add_f32 at ~190). Channel c uses the scale 2^s_c,
 //     s_c = 29 - ceil(log2 B_c), B_c = sum of |G * mask| over every (pixel, tap)
-//     accumulated so far: a bilinear corner weight is at most 1 and each (pixel,
+//     of the pass: a bilinear corner weight is at most 1 and each (pixel,
 //     tap) reaches a cell through at most one corner, so every cell sum stays
 //     below 2^29 (no overflow); each term is rounded to the unit 2^-s_c <= 2^-28 B_c.
-//     Integer sums are also order independent. When a pass of taps grows B_c,
-//     the values already held are shifted down to the new scale (rounded to
-//     nearest). The unit is relative to the tile's bound, not to each cell, so
+//     Integer sums are also order independent. The unit is relative to the pass's
+//     bound in the tile, not to each cell, so
 //     terms |G * mask| above 2^6 times the typical term of their (pass, channel)
 //     (gradient spikes: the bound would be theirs, and the quiet cells of the tile
 //     would be rounded at it) bypass the window: they go to global float atomics,
 //     and the bound covers the terms that stay. The typical term is 2 to the mean
-//     binary exponent of the 128 per-lane mean terms (a geometric mean, which a
-//     minority of spikes barely moves: each lane holds 2 pixels x the pass's taps).
+//     binary exponent of the per-lane mean terms (a geometric mean, which a
+//     minority of spikes barely moves: each lane holds 1 or 2 pixels x the pass's taps).
 //     In 3D a pass with spikes does not use the window. Neither does a pass with a
 //     non-finite bound (inf/nan must propagate as in the reference): it goes to
-//     global float atomics, after the window flushes what it holds.
-//     Corners outside the window go to global float atomics.
+//     global float atomics, as do corners outside the window.
 //   * The window (sampled-grid box around the tile's undeformed footprint plus a
-//     margin R per axis) accumulates over all passes of the tile and is flushed
-//     once: one float atomic per non-zero (cell, channel), 16 consecutive channels
-//     per cell.
+//     margin R per axis) is flushed at the end: one float atomic per non-zero
+//     (cell, channel), 16 consecutive channels per cell.
 #include "window.h"
 
 namespace tvdcn_hip {
@@ -62,9 +64,6 @@ namespace {
 
 using namespace win;
 
-constexpr int NW = 8;             // waves per workgroup (two per SIMD)
-constexpr int NT = 64 * NW;       // threads per workgroup
-constexpr int PB = 2;             // 16-pixel blocks per wave (NW * PB * 16 = BPX)
 constexpr int BM = 16;            // GEMM-side channels per K step
 // Fixed-point window: channel-major [16 c][cst], cst = window cells rounded so that
 // cst = 4 (mod 16). A scatter instruction's lanes are 16 pixels x 4 channel quads; the
@@ -81,14 +80,12 @@ constexpr int FIX_BITS = 29;      // fixed-point headroom: |cell sum| * 2^s_c < 
 // global memory, so the held value plus what went out stays the exact integer sum.
 constexpr int PREC_BITS = 26;
 constexpr unsigned WRAP_K = 0x78000000u;   // 2^31 - 2^27
-static_assert(NW * PB * 16 == BPX, "one tile of pixels per workgroup");
-static_assert(NT == BC * 32, "window rescale: 32 threads per channel");
 
 // LDS words ahead of the windows: geometry table [WIN_TMAX][BPX] x (position, mask),
-// per-wave channel bounds, scale exponents and flags, held bounds, rescale shifts (or
-// spike thresholds), largest terms, exponent statistics
+// per-wave channel bounds, scale exponents and flags, spike thresholds, largest terms,
+// exponent statistics
 constexpr int GEO_WORDS = WIN_TMAX * BPX * 4;
-constexpr int FIXED_WORDS = GEO_WORDS + NW * BC + 5 * BC + 4;
+constexpr int fixed_words(int nw) { return GEO_WORDS + nw * BC + 4 * BC + 4; }
 // a term above 2^SPIKE_BITS x 2^(mean exponent of the per-lane mean terms of its pass) is a spike
 constexpr int SPIKE_BITS = 6;
 
@@ -235,14 +232,17 @@ __device__ __forceinline__ unsigned row_sum16(unsigned v) {
     return row_reduce16(v, [](unsigned a, unsigned b) { return a + b; });
 }
 
-template <int DIM, typename T, bool SCATTER, bool COORD>
-__global__ void __launch_bounds__(NT)
+template <int DIM, typename T, bool SCATTER, bool COORD, int NW>
+__global__ void __launch_bounds__(64 * NW)
 bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wchunks, const uint16_t *zs,
                     const uint16_t *wsplit, const int *flag, const float *__restrict__ xcl,
                     const T *__restrict__ offset, const T *__restrict__ mask, float *__restrict__ gx_cl,
                     float *__restrict__ goff, float *__restrict__ gmask, const int gx_nchw) {
     constexpr int NC = 1 << DIM;
     constexpr int TMAX = WIN_TMAX;
+    constexpr int NT = 64 * NW;
+    constexpr int PB = BPX / (16 * NW);   // 16-pixel blocks per wave
+    static_assert(PB >= 1 && NW * PB * 16 == BPX, "one tile of pixels per workgroup");
     // scatter-only: the unit follows the largest kept term, cells sum modulo 2^32 (PREC_BITS)
     constexpr bool PREC = SCATTER && !COORD;
 
@@ -251,16 +251,12 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     float *bsum = smem + GEO_WORDS;                            // [NW][BC] partial bounds
     int *scl = reinterpret_cast<int *>(bsum + NW * BC);        // [BC] scale exponents, then the non-finite
                                                                // flag [BC] and the spike flag [BC + 1]
-    float *btot = bsum + NW * BC + BC + 4;                     // [BC] bound of what the window holds
-    int *shift = reinterpret_cast<int *>(btot + BC);           // [BC] rescale of the window for a pass
-    // [BC] spike thresholds of a pass with spikes, read before its rescale shifts are written (PREC
-    // sets both in one step and keeps no bound: the thresholds take the bound's words)
-    float *thr = PREC ? btot : reinterpret_cast<float *>(shift);
-    int *bmax = shift + BC;                                    // [BC] largest |G * mask| (float bits, >= 0)
+    float *thr = bsum + NW * BC + BC + 4;                      // [BC] spike thresholds of a pass with spikes
+    int *bmax = reinterpret_cast<int *>(thr + BC);             // [BC] largest |G * mask| (float bits, >= 0)
     unsigned *bexp = reinterpret_cast<unsigned *>(bmax + BC);  // [BC] exponent sums + (counts << 20)
     // (xg: the offset / mask gradients read X from global memory; no X window)
     const bool xg = COORD && wt.xglobal != 0;
-    float *xwin = smem + FIXED_WORDS;                          // [cells][XS] X window (COORD)
+    float *xwin = smem + fixed_words(NW);                          // [cells][XS] X window (COORD)
     int *iwin = reinterpret_cast<int *>(xwin + (COORD && !xg ? wt.cells * XS : 0));   // [BC][cst] fixed point
     const int cst = fix_stride(wt.cells);
     // [2][tpp][npiece][512] staged weight blocks of the 16-bit K loop (wt.wstage > 0)
@@ -276,6 +272,9 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     int L = xcd_remap(blockIdx.x, gridDim.x);
     const int ct = L % wt.c_tiles;
     L /= wt.c_tiles;
+    const int npass = (g.Kn + wt.tpp - 1) / wt.tpp;
+    const int t0 = L % npass * wt.tpp;
+    L /= npass;
     const int n_sp = g.B * wt.ntile[0] * wt.ntile[1] * wt.ntile[2];
     Tile tile;
     tile.init(g, wt, L % n_sp, ct, L / n_sp);
@@ -343,24 +342,21 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         }
     };
 
-    // ---- the fixed-point window accumulates over every pass of the tile and is flushed
-    //      once, at the end (or before a pass whose bound is not finite): one float atomic
-    //      per non-zero (cell, channel), 16 consecutive channels per cell (channels-last) or
-    //      32 consecutive cells per channel (gx_nchw)
-    bool win_data = false;   // the window holds accumulated values (uniform)
-    // thread = (channel tid % 16, cells tid / 16, + 32, ...) or, gx_nchw, (channel tid / 32, cells
-    // tid % 32, + 32, ...); FB cells' values are read before any is used (one LDS latency per
-    // batch). keep: the window is used again (cleared as read, barrier at the end); at the end
-    // of the workgroup neither is needed.
-    auto flush_window = [&](bool keep) {
+    // ---- the fixed-point window is flushed at the end: one float atomic per non-zero (cell,
+    //      channel), 16 consecutive channels per cell (channels-last) or STEP consecutive cells
+    //      per channel (gx_nchw)
+    // thread = (channel tid % 16, cells tid / 16, + STEP, ...) or, gx_nchw, (channel tid / STEP,
+    // cells tid % STEP, + STEP, ...); FB cells' values are read before any is used (one LDS
+    // latency per batch)
+    auto flush_window = [&]() {
         constexpr int FB = 8;
         constexpr int STEP = NT / 16;
-        static_assert(STEP == 32 && NT / 32 == BC, "both thread maps step 32 cells per channel");
-        const int c = gx_nchw ? tid >> 5 : tid & 15;
+        static_assert(NT / STEP == BC, "both thread maps step STEP cells per channel");
+        const int c = gx_nchw ? tid / STEP : tid & 15;
         const int se = scl[c];
         const bool c_ok = c0 + c < g.Cg;
         float *gbase = gxb + (size_t)(cg0 + c) * gcs;
-        const int first = gx_nchw ? tid & 31 : tid >> 4;
+        const int first = gx_nchw ? tid % STEP : tid >> 4;
         // cell walker (no divisions per cell), as in for_cells
         int lx = first % wt.WE[2];
         int rr = first / wt.WE[2];
@@ -393,18 +389,16 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
 #pragma unroll
             for (int j = 0; j < FB; ++j) {
                 if (iv[j] == 0) continue;
-                if (keep) iwin[c * cst + cell0 + j * STEP] = 0;   // cleared for what follows
                 if (si[j] >= 0) atomic_add(gbase + (size_t)si[j] * gps, ldexpf((float)iv[j], -se));
             }
         }
-        if (keep) __syncthreads();
     };
 
-    for (int t0 = 0; t0 < g.Kn; t0 += wt.tpp) {
+    {
         const int ntaps = min(wt.tpp, g.Kn - t0);
 
         // ---- sampling table of the pass, one (tap, pixel) per thread ------------------
-        fill_geo<DIM, T>(g, wt, tile, offset, mask, t0, ntaps, geo, tid, NT);
+        fill_geo<DIM, T, (WIN_TMAX * BPX + NT - 1) / NT>(g, wt, tile, offset, mask, t0, ntaps, geo, tid, NT);
 
         acc4 acc[TMAX][PB];
 #pragma unroll
@@ -529,6 +523,55 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
                     for (int k = 0; k < NP; ++k) zc[pb][k] = zn[pb][k];
             }
         };
+        // ---- the same with one weight fragment per tap, each reloaded for the next step as soon as
+        //      its MFMAs are issued: every load has a whole step to arrive (one-piece operands, whose
+        //      nine fragments fit beside sixteen waves' registers). Grids of a round or two of the chip
+        //      run at the latency of these loads
+        //      (16 taps on 256 -> 128 channels, 8 x 32x32, float16: 86 -> 83 us)
+        auto kloop16r = [&]() {
+            constexpr int NP = npiece_of<T>();
+            const int ms32 = wt.ms32;
+            const size_t zstep = (size_t)g.Pn * (NP * 32);
+            const uint16_t *zl[PB];
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb)
+                zl[pb] = zs + ((size_t)(b * g.G + grp) * ms32 * NP * g.Pn + (zp[pb] < 0 ? 0 : zp[pb])) * 32 + q * 8;
+            const uint16_t *wl = wsplit + ((size_t)(grp * wt.c_tiles + ct) * ms32 * g.Kn + t0) * (NP * 512) + lane * 8;
+            auto zfrag = [&](int st, uint4 (&f)[PB][NP]) {
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb)
+#pragma unroll
+                    for (int k = 0; k < NP; ++k)
+                        f[pb][k] = *reinterpret_cast<const uint4 *>(zl[pb] + (size_t)st * zstep + (size_t)k * g.Pn * 32);
+            };
+            auto wfrag = [&](int st, int tl, uint4 (&f)[NP]) {
+                const uint16_t *pw = wl + ((size_t)st * g.Kn + tl) * (NP * 512);
+#pragma unroll
+                for (int k = 0; k < NP; ++k) f[k] = *reinterpret_cast<const uint4 *>(pw + k * 512);
+            };
+            uint4 zc[PB][NP], zn[PB][NP], wr[TMAX][NP];
+            zfrag(0, zc);
+#pragma unroll
+            for (int tp = 0; tp < TMAX; ++tp)
+                if (tp < ntaps) wfrag(0, tp, wr[tp]);
+            for (int st = 0; st < ms32; ++st) {
+                const int stn = min(st + 1, ms32 - 1);
+                zfrag(stn, zn);
+                issue_fence();
+#pragma unroll
+                for (int tp = 0; tp < TMAX; ++tp) {
+                    if (tp >= ntaps) break;
+#pragma unroll
+                    for (int pb = 0; pb < PB; ++pb) acc[tp][pb] = mfma16x16x32_np<T, NP>(wr[tp], zc[pb], acc[tp][pb]);
+                    wfrag(stn, tp, wr[tp]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb)
+#pragma unroll
+                    for (int k = 0; k < NP; ++k) zc[pb][k] = zn[pb][k];
+            }
+        };
         // ---- 16-bit K loop with the weight blocks staged in LDS: a step's block (the pass's
         //      taps x NP pieces, 1 KB each, contiguous in the split layout) is the same for all
         //      eight waves; read straight from global memory it went eight times through the
@@ -602,8 +645,10 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         int use16 = __builtin_amdgcn_readfirstlane(use16_flag);
         asm volatile("" : "+s"(use16));
         if (use16) {
-            if (wt.wstage > 0)
+            if (DIM < 3 && wt.wstage > 0)   // (3D plans stage no weights)
                 kloop16s();
+            else if constexpr (NW == 16 && npiece_of<T>() == 1)
+                kloop16r();
             else
                 kloop16();
             if constexpr (npiece_of<T>() == 2) {
@@ -627,17 +672,15 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         }
         __syncthreads();   // geometry table (and X window) written
 
-        // ---- fixed-point scale per channel: the bound covers this pass plus everything
-        //      the window already holds; when it grows, the held values are shifted down
-        //      to the new (smaller or equal) scale. Terms above the spike threshold th of
-        //      their channel bypass the window and the bound.
+        // ---- fixed-point scale per channel. Terms above the spike threshold th of their
+        //      channel bypass the window and the bound.
         int sexp[4] = {0, 0, 0, 0};   // scale exponents of this lane's channels c0 + mq + v
         float th[4] = {0.f, 0.f, 0.f, 0.f};   // spike thresholds of this lane's channels
         bool use_window = false, spikes = false;
         if constexpr (SCATTER) {
             // first sweep: per-channel sum of the terms (a nan makes it non-finite), their
             // maximum, and over the lanes the sum of the biased exponents of the nonzero lane
-            // means + (their count << 20) (128 lanes of exponent < 2^8: no carry); otherwise
+            // means + (their count << 20) (256 lanes of exponent < 2^8: no carry); otherwise
             // the sum of the terms at or below lim[v]
             auto bound_sweep = [&](const float (&lim)[4], bool with_max) {
                 float part[4] = {0.f, 0.f, 0.f, 0.f}, pmax[4] = {0.f, 0.f, 0.f, 0.f};
@@ -697,38 +740,21 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
             };
             // scale of the pass from its (kept) bound bc, channel tid of wave 0's first 16 lanes
             auto set_scale = [&](float bc) {
-                const float tot = (win_data ? btot[tid] : 0.f) + bc;
                 // the pass uses the window only if every bound is finite (ballot over 16 lanes)
-                const unsigned long long bad = __ballot(!isfinite(tot));
+                const unsigned long long bad = __ballot(!isfinite(bc));
                 int e = 0;
-                if (tot > 0.f && isfinite(tot)) frexpf(tot, &e);   // tot < 2^e
-                shift[tid] = 0;
-                if (bad == 0ull) {
-                    if (win_data) shift[tid] = scl[tid] - (FIX_BITS - e);   // >= 0: the bound only grows
-                    scl[tid] = FIX_BITS - e;
-                    btot[tid] = tot;
-                }
+                if (bc > 0.f && isfinite(bc)) frexpf(bc, &e);   // bc < 2^e
+                scl[tid] = FIX_BITS - e;
                 if (tid == 0) scl[BC] = bad != 0ull;
             };
             // PREC: the scale of the pass from the largest term the window keeps (kmax; a pass
-            // with spikes keeps the terms up to their threshold), coarsened to what the window
-            // holds; bc (the sum of every term) only tells whether the pass is finite. A pass that
-            // skips the window (not finite; 3D with spikes: skip) leaves the held scale as it is:
-            // the window's flush reads it.
-            auto set_scale_prec = [&](float kmax, float bc, bool skip) {
+            // with spikes keeps the terms up to their threshold); bc (the sum of every term) only
+            // tells whether the pass is finite
+            auto set_scale_prec = [&](float kmax, float bc) {
                 const unsigned long long bad = __ballot(!isfinite(bc));
                 int e = 0;
-                if (kmax > 0.f) frexpf(kmax, &e);   // kmax < 2^e
-                int sc = PREC_BITS - e;
-                shift[tid] = 0;
-                if (bad == 0ull && !skip) {
-                    if (win_data) {
-                        const int held = scl[tid];
-                        sc = min(sc, held);
-                        shift[tid] = held - sc;
-                    }
-                    scl[tid] = sc;
-                }
+                if (kmax > 0.f && isfinite(kmax)) frexpf(kmax, &e);   // kmax < 2^e
+                scl[tid] = PREC_BITS - e;
                 if (tid == 0) scl[BC] = bad != 0ull;
             };
             const float no_lim[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
@@ -740,18 +766,16 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
                 for (int w = 0; w < NW; ++w) bc += bsum[w * BC + tid];
                 const unsigned es = bexp[tid];
                 const float big = __int_as_float(bmax[tid]);
-                bmax[tid] = 0;   // for the next pass (read after this pass's last barrier)
-                bexp[tid] = 0u;
                 // threshold 2^(mean unbiased exponent of the lane means + SPIKE_BITS), the mean
                 // rounded down (exact: integers below 2^24, a correctly rounded quotient of
-                // denominator <= 128 is an integer only when the true quotient is)
+                // denominator <= 256 is an integer only when the true quotient is)
                 const float cnt = (float)(es >> 20), esum = (float)(es & ((1u << 20) - 1u));
                 const float lim = cnt > 0.f ? ldexpf(1.f, (int)floorf(esum / cnt) - 127 + SPIKE_BITS) : INFINITY;
                 const bool spike = isfinite(bc) && big > lim;
                 thr[tid] = spike ? lim : INFINITY;
                 const unsigned long long any = __ballot(spike);
                 if constexpr (PREC)
-                    set_scale_prec(spike ? lim : big, bc, DIM == 3 && any != 0ull);
+                    set_scale_prec(spike ? lim : big, bc);
                 else if (any == 0ull)
                     set_scale(bc);   // no spike: the bound is final
                 if (tid == 0) scl[BC + 1] = any != 0ull;
@@ -783,28 +807,10 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
                 __syncthreads();
                 no_window = scl[BC] != 0;
             }
-            if (no_window) {
-                // not finite (or 3D spikes): what the window holds goes out at its scale, the
-                // pass goes to global float atomics (inf / nan propagate as in the reference)
-                if (win_data) flush_window(true);
-                win_data = false;
-                spikes = false;
-            } else {
-                if (win_data) {
-                    // rescale to nearest (halves up); a shift of 31 or more leaves at most a unit
-                    // (PREC: a held value may be anywhere in the 32-bit range)
-                    const int c = tid >> 5, sh = shift[c];
-                    if (sh > 0) {
-                        for (int cell = tid & 31; cell < cst; cell += 32) {
-                            const int v = iwin[c * cst + cell];
-                            iwin[c * cst + cell] = sh >= 31 ? 0 : (v >> sh) + ((v >> (sh - 1)) & 1);
-                        }
-                    }
-                    __syncthreads();
-                }
-                use_window = wt.cells > 0;
-                win_data = use_window;
-            }
+            // not finite (or 3D spikes): the pass goes to global float atomics (inf / nan propagate
+            // as in the reference)
+            if (no_window) spikes = false;
+            use_window = wt.cells > 0 && !no_window;
 #pragma unroll
             for (int v = 0; v < 4; ++v) sexp[v] = scl[mq + v];
         }
@@ -873,102 +879,138 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
                 if constexpr (DIM == 3) {
                     if (!SCATTER || use_window) {
                         // 3D: one branch-light path for every lane (window margins of about one
-                        // cell: most waves hold a lane with a corner outside the window)
+                        // cell: most waves hold a lane with a corner outside the window), the four
+                        // corners of each z plane in turn (a rolled loop: the plane's X and returned
+                        // values are all that is live at once, so that four waves fit a SIMD)
                         done = true;
-                        const Corners3 cr(g, wt, tile, r, deformable);
-                        if constexpr (COORD) {
-                            // G contracted with X per corner, then the trilinear / coordinate weights
-                            float gs = 0.f, gz = 0.f, gy = 0.f, gxx = 0.f;
+                        const Corners3M cr(g, wt, tile, r, deformable);
+                        const float fz = cr.fh[0], fy = cr.fh[1], fx = cr.fh[2];
+                        const float wyx[4] = {(1.f - fy) * (1.f - fx), (1.f - fy) * fx, fy * (1.f - fx), fy * fx};
+                        // G contracted with X per corner, then the trilinear / coordinate weights
+                        float gs = 0.f, gz = 0.f, gy = 0.f, gxx = 0.f;
+                        // (PREC: mask * G scaled, the corner weight <= 1 applied after, so no
+                        // intermediate leaves the float range)
+                        float gsc[4];
+                        if constexpr (SCATTER) {
 #pragma unroll
-                            for (int k = 0; k < 8; ++k) {
-                                if (k > 0 && !deformable) break;
-                                const acc4 x = corner_x3(g, wt, cr, k, xwin, mq, xb + mq, cq_ok, xg);
-                                const float gk = gv[0] * x[0] + gv[1] * x[1] + gv[2] * x[2] + gv[3] * x[3];
-                                const int bz = k >> 2, by = (k >> 1) & 1, bx = k & 1;
-                                const float wz = bz ? cr.fh[0] : 1.f - cr.fh[0];
-                                const float wy = by ? cr.fh[1] : 1.f - cr.fh[1];
-                                const float wx = bx ? cr.fh[2] : 1.f - cr.fh[2];
-                                gs += wz * wy * wx * gk;
-                                gz += (bz ? gk : -gk) * (wy * wx);
-                                gy += (by ? gk : -gk) * (wz * wx);
-                                gxx += (bx ? gk : -gk) * (wz * wy);
+                            for (int v = 0; v < 4; ++v) gsc[v] = ldexpf(PREC ? mk * gv[v] : gv[v], sexp[v]);
+                        }
+                        float *const gdst = gxb + (size_t)(cg0 + mq) * gcs;
+#pragma unroll 1
+                        for (int h = 0; h < 2; ++h) {
+                            if (h > 0 && !deformable) break;
+                            const unsigned wm = cr.wmask >> (4 * h), gm = cr.gmask >> (4 * h);
+                            const float wz = h ? fz : 1.f - fz;
+                            // window cell and grid index of the plane's corner j (y bit j / 2, x bit j % 2)
+                            const int cell_h = cr.cell0 + h * (wt.WE[1] * wt.WE[2]);
+                            const int idx_h = cr.idx0 + h * (g.S[1] * g.S[2]);
+                            auto cell_of = [&](int j) { return cell_h + (j >> 1) * wt.WE[2] + (j & 1); };
+                            auto idx_of = [&](int j) { return idx_h + (j >> 1) * g.S[2] + (j & 1); };
+                            if constexpr (COORD) {
+                                acc4 x[4];
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    x[j] = acc4{0.f, 0.f, 0.f, 0.f};
+                                    if (j > 0 && !deformable) continue;
+                                    if (!xg && ((wm >> j) & 1u))
+                                        x[j] = *reinterpret_cast<const acc4 *>(xwin + cell_of(j) * XS + mq);
+                                    else if (cq_ok && ((gm >> j) & 1u))
+                                        x[j] = *reinterpret_cast<const acc4 *>(xb + mq + (size_t)idx_of(j) * g.C);
+                                }
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    if (j > 0 && !deformable) break;
+                                    const float gk = gv[0] * x[j][0] + gv[1] * x[j][1] + gv[2] * x[j][2] + gv[3] * x[j][3];
+                                    const float wy = (j >> 1) ? fy : 1.f - fy, wx = (j & 1) ? fx : 1.f - fx;
+                                    gs += wz * wyx[j] * gk;
+                                    gz += (h ? gk : -gk) * wyx[j];
+                                    gy += ((j >> 1) ? gk : -gk) * (wz * wx);
+                                    gxx += ((j & 1) ? gk : -gk) * (wz * wy);
+                                }
                             }
+                            if constexpr (SCATTER) {
+                                if (!cq_ok) continue;
+                                // (PREC) the returned old values of the plane's corners are checked for a
+                                // possible wrap, the adds recomputed where one is
+                                unsigned near = 0u;
+                                unsigned old[4][4];
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    if (j > 0 && !deformable) break;
+                                    if (!((gm >> j) & 1u)) continue;
+                                    const float cw = wz * wyx[j];
+                                    const float sw = mk * cw;
+                                    if ((wm >> j) & 1u) {
+                                        unsigned int *dst = reinterpret_cast<unsigned int *>(iwin + mq * cst + cell_of(j));
+#pragma unroll
+                                        for (int v = 0; v < 4; ++v) {
+                                            if constexpr (PREC) {
+                                                old[j][v] = atomicAdd(dst + v * cst, (unsigned int)fixed_round(cw * gsc[v]));
+                                                near = max(near, old[j][v] + WRAP_K);
+                                            } else {
+                                                atomicAdd(dst + v * cst, (unsigned int)fixed_round(sw * gsc[v]));
+                                            }
+                                        }
+                                    } else {
+                                        float *dst = gdst + (size_t)idx_of(j) * gps;
+#pragma unroll
+                                        for (int v = 0; v < 4; ++v) atomic_add(dst + v * gcs, sw * gv[v]);
+                                    }
+                                }
+                                if (PREC && near >= 2u * WRAP_K) {
+                                    // some add may have wrapped: its 2^32 units go to global memory
+#pragma unroll
+                                    for (int j = 0; j < 4; ++j) {
+                                        if (j > 0 && !deformable) break;
+                                        if (!((gm >> j) & (wm >> j) & 1u)) continue;
+                                        const float cw = wz * wyx[j];
+#pragma unroll
+                                        for (int v = 0; v < 4; ++v) {
+                                            const float spl = wrap_spill(old[j][v], fixed_round(cw * gsc[v]), sexp[v]);
+                                            if (spl != 0.f) atomic_add(gdst + (size_t)idx_of(j) * gps + v * gcs, spl);
+                                        }
+                                    }
+                                }
+                            }
+                        }
+                        if constexpr (COORD) {
                             qv[0] = mk * gz;
                             qv[1] = mk * gy;
                             qv[2] = mk * gxx;
                             qv[3] = cr.inside ? gs : 0.f;
                         }
-                        if constexpr (SCATTER) {
-                            if (cq_ok) {
-                                // (PREC: mask * G scaled, the corner weight <= 1 applied after, so no
-                                // intermediate leaves the float range)
-                                float gsc[4];
+                    } else {
+                        // the pass scatters to global memory (not finite, or spikes): every corner in
+                        // turn, X contracted with the weights before G (inf / nan as in the reference)
+                        done = true;
+                        const AxisW<DIM, float> aw = record_weights<DIM>(g, r, deformable);
+                        acc4 d[DIM], sv = acc4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                                for (int v = 0; v < 4; ++v) gsc[v] = ldexpf(PREC ? mk * gv[v] : gv[v], sexp[v]);
-                                float *gdst = gxb + (size_t)(cg0 + mq) * gcs;
-                                if constexpr (!PREC) {
+                        for (int a = 0; a < DIM; ++a) d[a] = acc4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                                    for (int k = 0; k < 8; ++k) {
-                                        if (k > 0 && !deformable) break;
-                                        if (!cr.in_grid(k)) continue;
-                                        const float sw = mk * cr.weight(k);
-                                        if (cr.in_win(k)) {
-                                            unsigned int *dst = reinterpret_cast<unsigned int *>(iwin + mq * cst + cr.cell(wt, k));
+                        for (int k = 0; k < NC; ++k) {
+                            int idx;
+                            bool v;
+                            corner_at<DIM, float>(g, aw, k, idx, v);
+                            const float w = v ? corner_weight<DIM, float>(aw, k) : 0.f;
+                            if constexpr (COORD) {
+                                acc4 x = acc4{0.f, 0.f, 0.f, 0.f};
+                                if (v && cq_ok) x = *reinterpret_cast<const acc4 *>(xb + (size_t)idx * g.C + mq);
 #pragma unroll
-                                            for (int v = 0; v < 4; ++v)
-                                                atomicAdd(dst + v * cst, (unsigned int)fixed_round(sw * gsc[v]));
-                                        } else {
-                                            float *dst = gdst + (size_t)cr.idx(g, k) * gps;
-#pragma unroll
-                                            for (int v = 0; v < 4; ++v) atomic_add(dst + v * gcs, sw * gv[v]);
-                                        }
-                                    }
-                                } else {
-                                    // the returned old values of four corners at a time are checked for a
-                                    // possible wrap, the adds recomputed where one is
-#pragma unroll
-                                    for (int h = 0; h < 2; ++h) {
-                                        if (h > 0 && !deformable) break;
-                                        unsigned near = 0u;
-                                        unsigned old[4][4];
-#pragma unroll
-                                        for (int j = 0; j < 4; ++j) {
-                                            const int k = 4 * h + j;
-                                            if (k > 0 && !deformable) break;
-                                            if (!cr.in_grid(k)) continue;
-                                            if (cr.in_win(k)) {
-                                                unsigned int *dst = reinterpret_cast<unsigned int *>(iwin + mq * cst + cr.cell(wt, k));
-                                                const float sw = cr.weight(k);
-#pragma unroll
-                                                for (int v = 0; v < 4; ++v) {
-                                                    old[j][v] = atomicAdd(dst + v * cst, (unsigned int)fixed_round(sw * gsc[v]));
-                                                    near = max(near, old[j][v] + WRAP_K);
-                                                }
-                                            } else {
-                                                float *dst = gdst + (size_t)cr.idx(g, k) * gps;
-                                                const float sw = mk * cr.weight(k);
-#pragma unroll
-                                                for (int v = 0; v < 4; ++v) atomic_add(dst + v * gcs, sw * gv[v]);
-                                            }
-                                        }
-                                        if (near >= 2u * WRAP_K) {
-                                            // some add may have wrapped: its 2^32 units go to global memory
-#pragma unroll
-                                            for (int j = 0; j < 4; ++j) {
-                                                const int k = 4 * h + j;
-                                                if (k > 0 && !deformable) break;
-                                                if (!cr.in_grid(k) || !cr.in_win(k)) continue;
-                                                const float sw = cr.weight(k);
-#pragma unroll
-                                                for (int v = 0; v < 4; ++v) {
-                                                    const float sp = wrap_spill(old[j][v], fixed_round(sw * gsc[v]), sexp[v]);
-                                                    if (sp != 0.f) atomic_add(gdst + (size_t)cr.idx(g, k) * gps + v * gcs, sp);
-                                                }
-                                            }
-                                        }
-                                    }
-                                }
+                                for (int a = 0; a < DIM; ++a) d[a] += corner_dweight<DIM, float>(aw, k, a) * x;
+                                if (aw.inside) sv += w * x;
                             }
+                            if (v && cq_ok) {
+                                float *dst = gxb + (size_t)(cg0 + mq) * gcs + (size_t)idx * gps;
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) atomic_add(dst + u * gcs, mk * w * gv[u]);
+                            }
+                        }
+                        if constexpr (COORD) {
+#pragma unroll
+                            for (int a = 0; a < DIM; ++a)
+                                qv[a] = mk * (gv[0] * d[a][0] + gv[1] * d[a][1] + gv[2] * d[a][2] + gv[3] * d[a][3]);
+                            qv[DIM] = gv[0] * sv[0] + gv[1] * sv[1] + gv[2] * sv[2] + gv[3] * sv[3];
                         }
                     }
                 } else if (fc >= 0 && (!SCATTER || use_window) && !lane_spike) {
@@ -1064,7 +1106,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
                         }
                     }
                 }
-                if (!done) {
+                if (DIM < 3 && !done) {
                     // general path: per-corner validity, window membership and global fallback
                     // (also taken by fast records when the pass scatters to global memory)
                     const AxisW<DIM, float> aw = record_weights<DIM>(g, record_position<DIM>(wt, tile, r), deformable);
@@ -1181,10 +1223,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         __syncthreads();   // all waves done with the geometry table and the window
 
         // ---- after the last pass, the window goes out
-        if (SCATTER && win_data && t0 + wt.tpp >= g.Kn) {
-            flush_window(false);   // the workgroup's last use of the window
-            win_data = false;
-        }
+        if (SCATTER && use_window) flush_window();
     }
 }
 
@@ -1289,28 +1328,43 @@ data_prep_kernel(const T *__restrict__ z, uint16_t *__restrict__ zs, const T *__
 }
 
 template <bool SCATTER, bool COORD> size_t lds_bytes(const WinTiles &t) {
-    return ((size_t)FIXED_WORDS + (SCATTER ? (size_t)BC * fix_stride(t.cells) : 0) +
+    return ((size_t)fixed_words(t.waves) + (SCATTER ? (size_t)BC * fix_stride(t.cells) : 0) +
             (COORD && !t.xglobal ? (size_t)t.cells * XS : 0)) *
                sizeof(float) +
            (size_t)t.wstage;
+}
+
+template <int DIM, typename T, bool SCATTER, bool COORD, int NW>
+hipError_t launch_w(const Geo &g, const WinTiles &tl, const void *z, const void *wchunks, const void *zs,
+                    const void *wsplit, const int *flag, const void *xcl, const void *offset, const void *mask,
+                    void *gx_cl, void *goff, void *gmask, hipStream_t s, bool gx_nchw) {
+    auto kern = bwd_data_win_kernel<DIM, T, SCATTER, COORD, NW>;
+    const size_t lds = lds_bytes<SCATTER, COORD>(tl);
+    static std::atomic<unsigned long long> lds_raised{0};   // per device, see raise_lds_limit
+    if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
+        return e;
+    const long long blocks = (long long)g.G * g.B * tl.ntile[0] * tl.ntile[1] * tl.ntile[2] * tl.c_tiles * ((g.Kn + tl.tpp - 1) / tl.tpp);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * NW), lds, s, g, tl, static_cast<const T *>(z),
+                       static_cast<const float *>(wchunks), static_cast<const uint16_t *>(zs),
+                       static_cast<const uint16_t *>(wsplit), flag, static_cast<const float *>(xcl),
+                       static_cast<const T *>(offset), static_cast<const T *>(mask), static_cast<float *>(gx_cl),
+                       static_cast<float *>(goff), static_cast<float *>(gmask), gx_nchw ? 1 : 0);
+    return hipGetLastError();
 }
 
 template <int DIM, typename T, bool SCATTER, bool COORD>
 hipError_t launch_k(const Geo &g, const WinTiles &tl, const void *z, const void *wchunks, const void *zs,
                     const void *wsplit, const int *flag, const void *xcl, const void *offset, const void *mask,
                     void *gx_cl, void *goff, void *gmask, hipStream_t s, bool gx_nchw) {
-    auto kern = bwd_data_win_kernel<DIM, T, SCATTER, COORD>;
-    const size_t lds = lds_bytes<SCATTER, COORD>(tl);
-    static std::atomic<unsigned long long> lds_raised{0};   // per device, see raise_lds_limit
-    if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
-        return e;
-    const long long blocks = (long long)g.G * g.B * tl.ntile[0] * tl.ntile[1] * tl.ntile[2] * tl.c_tiles;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NT), lds, s, g, tl, static_cast<const T *>(z),
-                       static_cast<const float *>(wchunks), static_cast<const uint16_t *>(zs),
-                       static_cast<const uint16_t *>(wsplit), flag, static_cast<const float *>(xcl),
-                       static_cast<const T *>(offset), static_cast<const T *>(mask), static_cast<float *>(gx_cl),
-                       static_cast<float *>(goff), static_cast<float *>(gmask), gx_nchw ? 1 : 0);
-    return hipGetLastError();
+    if (tl.waves == 16)
+        return launch_w<DIM, T, SCATTER, COORD, 16>(g, tl, z, wchunks, zs, wsplit, flag, xcl, offset, mask, gx_cl, goff,
+                                                    gmask, s, gx_nchw);
+    // (3D plans always take sixteen waves)
+    if constexpr (DIM < 3)
+        if (tl.waves == 8)
+            return launch_w<DIM, T, SCATTER, COORD, 8>(g, tl, z, wchunks, zs, wsplit, flag, xcl, offset, mask, gx_cl,
+                                                       goff, gmask, s, gx_nchw);
+    return hipErrorInvalidValue;
 }
 
 template <int DIM, typename T>
@@ -1466,15 +1520,20 @@ WinTiles plan_data_win(const Geo &g, int dtype, int dim, bool scatter, bool coor
     t.lbxy = ilog2(box[1] * box[2]);
     t.c_tiles = (g.Cg + BC - 1) / BC;
     t.m_steps = (g.Mg + BM - 1) / BM;
+    const int npass = (g.Kn + WIN_TMAX - 1) / WIN_TMAX;
+    t.tpp = (g.Kn + npass - 1) / npass;
+    // eight waves share each weight fragment's read between two pixel blocks, which the K loop of a
+    // large grid needs; sixteen hide more latency, which bounds grids of up to two rounds of the
+    // chip (one workgroup per CU) and the 3D epilogue
+    const long long blocks = (long long)g.G * g.B * t.ntile[0] * t.ntile[1] * t.ntile[2] * t.c_tiles * npass;
+    t.waves = dim == 3 || blocks <= 512 ? 16 : 8;
     // per window cell: the fixed-point accumulators (scatter) and / or the X values
     // (offset/mask gradients), as the launches this plan serves need them
     // (+ BC * 16 words: the fixed-point window's stride rounding)
-    const size_t fixed = (FIXED_WORDS + (scatter ? BC * 16 : 0)) * sizeof(float);
+    const size_t fixed = (fixed_words(t.waves) + (scatter ? BC * 16 : 0)) * sizeof(float);
     const size_t cell = ((scatter ? BC : 0) + (coord ? XS : 0)) * sizeof(float);
     const WinTiles base = t;
     t = win_resize(base, g, dim, fixed, cell);
-    const int npass = (g.Kn + WIN_TMAX - 1) / WIN_TMAX;
-    t.tpp = (g.Kn + npass - 1) / npass;
     t.npiece = dtype == kF32 ? 2 : 1;
     // 1D / 2D passes of nine taps: the K loop's weight blocks staged in LDS when the window
     // keeps a margin of min(R, 4) cells beside the buffers (3D: short K loops, and the window
