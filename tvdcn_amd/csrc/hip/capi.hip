@@ -90,7 +90,8 @@ struct Plan {
 bool fits_int(int64_t v) { return v >= 0 && v <= (int64_t)INT_MAX; }
 
 // Plan of one batch block of `batch` images (the descriptor's other fields as given).
-tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch) {
+// (lean: the forward plan without partial sums in the workspace)
+tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch, bool lean = false) {
     tvdcn_status st = output_size(d, pl.out_size);
     if (st) return st;
     if (d->dtype < 0 || d->dtype > 3) return fail(TVDCN_STATUS_INVALID_ARGUMENT, "unknown dtype");
@@ -205,7 +206,7 @@ tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch) {
                                weight_win_fixed_bytes(g, pl.dim, pl.wn_s.tpp, pl.dtype == kF32 ? 2 : 1),
                                x_window_cell_bytes());
     pl.ww = plan_weight_win(g, pl.wn_w, pl.dim);
-    pl.fw = plan_fwd_win(g, pl.wn_s, pl.dim, pl.wn_f);
+    pl.fw = plan_fwd_win(g, pl.wn_s, pl.dim, pl.wn_f, lean);
     const bool cl_in = (d->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
     // (1D only: there a window row is the tile's 256 pixels + margins, whole lines of each channel;
     // 2D / 3D window rows are 10-26 cells, and the flush and out-of-window corners then reach
@@ -324,9 +325,9 @@ Layout layout(const Plan &pl, bool backward) {
     auto take_w16 = [&]() {
         if (pl.fw.ok && pl.fw.w16_elems) L.w16 = take(align_up(pl.fw.w16_elems * 2));
     };
-    // fp32 output of a slice-split windowed forward when the output dtype is not fp32
-    const bool split_acc = pl.fw.ok && pl.fw.ksplit > 1 && pl.dtype != kF32;
-    const size_t yacc_bytes = align_up((size_t)g.B * g.M * g.Pn * sizeof(float));
+    // the fp32 partials of a windowed forward in shares
+    const bool split_acc = pl.fw.ok && pl.fw.ksplit > 1;
+    const size_t yacc_bytes = align_up((size_t)pl.fw.ksplit * g.B * g.M * g.Pn * sizeof(float));
     if (!backward) {
         if (!pl.transposed) {
             L.xcl = take(cl_bytes);
@@ -549,10 +550,8 @@ tvdcn_status forward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const 
     if (!pl.transposed) {
         void *xcl = at(workspace, L.xcl), *wf = at(workspace, L.wf);
         void *w16 = pl.fw.ok && sampled16_host_ok(pl, desc) ? at(workspace, L.w16) : nullptr;
-        // the flag and (split channel slices) the fp32 accumulator zeroed by one launch
-        void *y32 = pl.fw.ok && pl.fw.ksplit > 1 ? (dt == kF32 ? output : at(workspace, L.yacc)) : nullptr;
-        const FillItem fills[2] = {{flag, 4 * OPERAND_FLAG_WORDS}, {y32, y32 ? (size_t)g.B * g.M * g.Pn * 4 : 0}};
-        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 2, s));
+        const FillItem fills[1] = {{flag, 4 * OPERAND_FLAG_WORDS}};
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 1, s));
         const void *x_in_place = nullptr;
         // the 16-bit loop's mask range check and (fp32) its operands' largest magnitudes ride on the
         // input's layout copy when there is one
@@ -581,9 +580,7 @@ tvdcn_status forward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const 
             }
             TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
                          launch_fwd_win(dt, pl.dim, g, pl.wn_f, pl.fw, xcl, wf, w16, flag, offset, mask, bias, output,
-                                        y32, s));
-            if (pl.fw.ksplit > 1 && dt != kF32)
-                TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_acc_to_storage(dt, y32, output, (size_t)g.B * g.M * g.Pn, s));
+                                        at(workspace, L.yacc), s));
         } else {
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_weight_fwd_layout(dt, g, weight, wf, pl.ft.Mg_pad, pl.ft.Cg_pad, s));
             TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
@@ -639,17 +636,13 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         // conv: grad_input accumulated in place (channels-last of the accumulation type, or the
         // float32 (B, C, *S) tensor on the windowed data gradient), else a channels-last accumulator
         void *gx_cl = pl.transposed ? nullptr : pl.gx_in_place ? grad_input : at(workspace, L.cl_acc);
-        // transposed, input gradient on the split forward plan: its fp32 accumulator
-        void *y32 = pl.transposed && pl.fw.ok && pl.fw.ksplit > 1 ? (dt == kF32 ? grad_input : at(workspace, L.yacc))
-                                                                   : nullptr;
-        // the offset / mask gradient accumulators, the operand flag, grad_input (conv) or the split
-        // accumulator (transposed) zeroed by one launch
-        const FillItem fills[5] = {{goff, goff ? n_goff * ab : 0},
+        // the offset / mask gradient accumulators, the operand flag and grad_input (conv) zeroed by one
+        // launch
+        const FillItem fills[4] = {{goff, goff ? n_goff * ab : 0},
                                    {gmask, gmask ? n_gmask * ab : 0},
                                    {flag, 4 * OPERAND_FLAG_WORDS},
-                                   {gx_cl, gx_cl ? (size_t)g.B * g.Sn * g.C * ab : 0},
-                                   {y32, y32 ? (size_t)g.B * g.M * g.Pn * 4 : 0}};
-        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 5, s));
+                                   {gx_cl, gx_cl ? (size_t)g.B * g.Sn * g.C * ab : 0}};
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 4, s));
         const bool coord = offset != nullptr || mask != nullptr;
         // the 16-bit loops of the sampled side (weight gradient; transposed: input gradient)
         const bool sampled16 = sampled16_host_ok(pl, desc) && (pl.ww.ok || (pl.transposed && pl.fw.ok));
@@ -726,10 +719,7 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
                     TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fwd_win_layout(dt, g, pl.fw, weight, wf, s));
                 TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
                              launch_fwd_win(dt, pl.dim, g, pl.wn_f, pl.fw, xcl, wf, w16, flag, offset, mask, nullptr,
-                                            grad_input, y32, s));
-                if (pl.fw.ksplit > 1 && dt != kF32)
-                    TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
-                                 launch_acc_to_storage(dt, y32, grad_input, (size_t)g.B * g.M * g.Pn, s));
+                                            grad_input, at(workspace, L.yacc), s));
             } else {
                 TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_weight_fwd_layout(dt, g, weight, wf, pl.ft.Mg_pad, pl.ft.Cg_pad, s));
                 TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
@@ -767,16 +757,16 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
 }
 
 // Workspace bytes of a call: the largest of its blocks' layouts (a full block and the remainder).
-size_t workspace_bytes_of(const tvdcn_conv_desc *desc, bool backward) {
+size_t workspace_bytes_of(const tvdcn_conv_desc *desc, bool backward, bool lean = false) {
     int64_t block = 0;
     if (batch_block(desc, block)) return 0;
     Plan pl;
-    if (make_plan(desc, pl, block)) return 0;
+    if (make_plan(desc, pl, block, lean)) return 0;
     size_t n = layout(pl, backward).total;
     const int64_t tail = block > 0 ? desc->batch % block : 0;
     if (tail > 0) {
         Plan pt;
-        if (make_plan(desc, pt, tail)) return 0;
+        if (make_plan(desc, pt, tail, lean)) return 0;
         n = std::max(n, layout(pt, backward).total);
     }
     return n;
@@ -785,7 +775,7 @@ size_t workspace_bytes_of(const tvdcn_conv_desc *desc, bool backward) {
 // The forward over the batch blocks (pointers checked, workspace large enough).
 tvdcn_status forward_blocks(const tvdcn_conv_desc *desc, int64_t block, const void *input, const void *weight,
                             const void *offset, const void *mask, const void *bias, void *output, void *workspace,
-                            void *stream) {
+                            void *stream, bool lean = false) {
     ImageElems ie;
     int64_t blk = 0;
     tvdcn_status st = batch_block(desc, blk, &ie);
@@ -797,7 +787,7 @@ tvdcn_status forward_blocks(const tvdcn_conv_desc *desc, int64_t block, const vo
     for (int64_t b0 = 0; b0 < desc->batch; b0 += block) {
         const int64_t nb = std::min<int64_t>(block, desc->batch - b0);
         Plan pl;
-        st = make_plan(desc, pl, nb);
+        st = make_plan(desc, pl, nb, lean);
         if (st) return st;
         st = forward_planned(pl, desc, adv(input, b0 * ie.in * es), weight, adv(offset, b0 * ie.offset * es),
                              adv(mask, b0 * ie.mask * es), bias, adv(output, b0 * ie.out * es), workspace, stream);
@@ -902,7 +892,9 @@ tvdcn_status tvdcn_deform_conv_forward_noalloc(const tvdcn_conv_desc *desc, cons
     if (st) return st;
     st = check_aligned({input, weight, offset, mask, bias, output});
     if (st) return st;
-    const size_t need = workspace_bytes_of(desc, false);
+    // (partial sums are taken only where the scratch array has room for them)
+    const bool lean = workspace_bytes_of(desc, false) > (size_t)TVDCN_SCRATCH_BYTES;
+    const size_t need = workspace_bytes_of(desc, false, lean);
     if (need > (size_t)TVDCN_SCRATCH_BYTES)
         return fail(TVDCN_STATUS_WORKSPACE_TOO_SMALL,
                     "forward_noalloc: this problem needs " + std::to_string(need) +
@@ -912,7 +904,7 @@ tvdcn_status tvdcn_deform_conv_forward_noalloc(const tvdcn_conv_desc *desc, cons
     void *ws = nullptr;
     st = scratch_of_current_device(&ws);
     if (st) return st;
-    return forward_blocks(desc, block, input, weight, offset, mask, bias, output, ws, stream);
+    return forward_blocks(desc, block, input, weight, offset, mask, bias, output, ws, stream, lean);
 }
 
 tvdcn_status tvdcn_deform_conv_backward(const tvdcn_conv_desc *desc, const void *grad_out, const void *input,

@@ -116,6 +116,22 @@ __device__ __forceinline__ Vec4<A> load4_t(const T *p) {
     }
 }
 
+// the matching store
+template <typename T, typename A>
+__device__ __forceinline__ void store4_t(T *p, const Vec4<A> &v) {
+    if constexpr (sizeof(T) == sizeof(A)) {
+        store4<A>(reinterpret_cast<A *>(p), v);
+    } else {
+        uint2 u;
+        T *h = reinterpret_cast<T *>(&u);
+        h[0] = from_acc<T, A>(v.x);
+        h[1] = from_acc<T, A>(v.y);
+        h[2] = from_acc<T, A>(v.z);
+        h[3] = from_acc<T, A>(v.w);
+        *reinterpret_cast<uint2 *>(p) = u;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // MFMA 16x16x4 (fp32 and fp64). Operand layout, lane l of 64:
 //   A[i][k]: i = l % 16, k = l / 16      B[k][j]: j = l % 16, k = l / 16

@@ -8,7 +8,8 @@
 // deform_conv2d_kernel.cpp:341-380; 1D/3D twins); the columns are never written
 // to HBM. Also computes the transposed op's input gradient.
 //
-// Workgroup = (spatial tile of 256 column pixels, 128 or 64 GEMM-side rows); eight
+// Workgroup = (spatial tile of 256 column pixels, 128 or 64 GEMM-side rows, a share of the (pass,
+// channel slice) units: grids too small to fill the chip take several shares); eight
 // waves, wave w owning 32 pixels x all rows (64 or 32 accumulators per lane; 64-row
 // tiles serve small GEMM sides and grids too small to fill the chip). The reduction runs
 // over 16-channel slices x taps; per step (slice, tap) every lane forms its own MFMA
@@ -62,7 +63,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     int L = xcd_remap(blockIdx.x, gridDim.x);
     const int mt = L % fw.m_tiles;
     L /= fw.m_tiles;
-    const int ks = L % fw.ksplit;   // share of the channel slices (fw.ksplit == 2: fp32 partials in y32)
+    const int ks = L % fw.ksplit;   // share of the (pass, channel slice) units (fw.ksplit > 1: fp32 partials)
     L /= fw.ksplit;
     const int n_sp = g.B * wt.ntile[0] * wt.ntile[1] * wt.ntile[2];
     const int sp = L % n_sp;
@@ -77,7 +78,15 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // the sampling table's masks carry 2^s_b, so that the B fragments come out of the sampling at
     // their pieces' scale
     const float mscale_b = ldexpf(1.f, s_b);
-    const int cs_lo = ks * fw.slices_per, cs_hi = min(slices, cs_lo + fw.slices_per);
+    // this share's units u = pass * slices + slice, u in [u_lo, u_lo + fw.units_per); per pass the slices
+    // [cs_lo, cs_hi) of them
+    const int u_lo = ks * fw.units_per;
+    int cs_lo = 0, cs_hi = 0;
+    auto pass_slices = [&](int pass) {
+        cs_lo = max(u_lo - pass * slices, 0);
+        cs_hi = min(u_lo + fw.units_per - pass * slices, slices);
+        return cs_lo < cs_hi;
+    };
 
     Tile tile;
     tile.init(g, wt, sp, 0, grp);
@@ -423,7 +432,8 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 for (int k = 0; k < NP; ++k) f[k] = *reinterpret_cast<const uint4 *>(p + lane * 8 + k * 512);
             };
             static_assert(MB % 2 == 0, "row blocks in pairs: the next step's block 0 lands in slot 0");
-            for (int t0 = 0; t0 < g.Kn; t0 += wt.tpp) {
+            for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
+                if (!pass_slices(pass)) continue;
                 const int ntaps = min(wt.tpp, g.Kn - t0);
                 const int ngr = (ntaps + 3) >> 2;
                 const int ngroups = (cs_hi - cs_lo) * ngr;
@@ -479,7 +489,8 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 }
             }
         } else {
-            for (int t0 = 0; t0 < g.Kn; t0 += wt.tpp) {
+            for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
+                if (!pass_slices(pass)) continue;
                 const int ntaps = min(wt.tpp, g.Kn - t0);
                 const int ngr = (ntaps + 3) >> 2;   // tap groups per slice
                 const int ngroups = (cs_hi - cs_lo) * ngr;
@@ -524,9 +535,11 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
             }
         }
     } else if (use16_flag) {
-        for (int t0 = 0; t0 < g.Kn; t0 += wt.tpp) pass16(t0, min(wt.tpp, g.Kn - t0));
+        for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass)
+            if (pass_slices(pass)) pass16(t0, min(wt.tpp, g.Kn - t0));
     } else {
-        for (int t0 = 0; t0 < g.Kn; t0 += wt.tpp) {
+        for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
+            if (!pass_slices(pass)) continue;
             const int ntaps = min(wt.tpp, g.Kn - t0);
             const int nsteps = (cs_hi - cs_lo) * ntaps;
             geo_og = geo_mg = -1;   // a new pass of taps: the table must be rebuilt
@@ -566,9 +579,9 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
         }
     }
 
-    // ---- epilogue: + bias, store NC<spatial>. With two slice shares, each adds its fp32
-    //      partial to y32 (zeroed by the caller; bias with the first share): a sum of two
-    //      terms onto zero is the same in either order, so the result is deterministic.
+    // ---- epilogue: + bias, store NC<spatial>. With several shares each stores its fp32 partial
+    //      to its own plane of y32 (bias with the first share); share_sum_kernel adds the planes in
+    //      order, so the result is deterministic.
 #pragma unroll
     for (int pb = 0; pb < PB; ++pb) {
         const int p = tile.pixel(g, wt, wave * (PB * 16) + pb * 16 + (lane & 15));
@@ -586,9 +599,30 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                     if (fw.ksplit == 1)
                         y[o] = from_acc<T, float>(r);
                     else
-                        atomic_add(y32 + o, r);
+                        y32[(size_t)ks * g.B * g.M * g.Pn + o] = r;
                 }
             }
+    }
+}
+
+// y[i] = sum over the shares k of part[k][i], in order (n values per share). VEC: 16-byte loads
+// (n % 4 == 0). Bound by the partials' bytes, read once each.
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256) share_sum_kernel(const float *__restrict__ part, T *__restrict__ y, size_t n,
+                                                        int shares) {
+    constexpr int W = VEC ? 4 : 1;
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * W;
+    if (i >= n) return;
+    if constexpr (VEC) {
+        acc4 v = *reinterpret_cast<const acc4 *>(part + i);
+#pragma unroll 4
+        for (int k = 1; k < shares; ++k) v += *reinterpret_cast<const acc4 *>(part + (size_t)k * n + i);
+        store4_t<T, float>(y + i, Vec4<float>{v[0], v[1], v[2], v[3]});
+    } else {
+        float v = part[i];
+#pragma unroll 4
+        for (int k = 1; k < shares; ++k) v += part[(size_t)k * n + i];
+        y[i] = from_acc<T, float>(v);
     }
 }
 
@@ -713,20 +747,66 @@ hipError_t launch_d(int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw,
 
 size_t x_window_cell_bytes() { return XS * sizeof(float); }
 
-FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt) {
+// Rows per workgroup and shares of the (pass, channel slice) units, from a model of the launch's time:
+// one workgroup per CU at a time (the window takes most of the LDS), so `rounds` of the chip, each a
+// start and a table fill plus the share's units, then the sum of the partials. Microseconds, measured
+// on one to eight units of 5 tap pairs and 16 to 256 workgroups: a unit takes about the same with 64
+// rows as with 128, so the larger tile wins unless the GEMM side is small, and a grid that leaves
+// CUs idle takes more shares instead. Inference, us a call, against 64-row tiles in at most two
+// shares: float16 256 -> 256 channels k3 on one 25 x 38 image (48 workgroups of 8 units -> 192 of
+// 1) 110 -> 58; bfloat16 128 -> 128 on 2 x 100 x 152 (280 of 8, two rounds -> 140 of 128 rows)
+// 177 -> 127; float16 3D 32 -> 32 k3 on 9 x 28 x 30 (96 of 4 passes -> 192 of 2) 91 -> 61.
+namespace {
+constexpr double SHARE_US = 8.0, PAIR_US = 2.0, SUM_US = 5.0, SUM_BYTES_PER_US = 4e6;
+constexpr size_t SHARE_BYTES_MAX = (size_t)64 << 20;   // partials of one call
+void split_shares(FwdWin &f, const Geo &g, int mb_max, long long spatial, int slices, int tpp, int npiece, bool lean) {
+    const int npass = (g.Kn + tpp - 1) / tpp, units = npass * slices;
+    const double out_bytes = 4.0 * g.B * g.M * g.Pn;
+    double best = 0.0;
+    for (int mb = mb_max; mb >= 4; mb -= 4) {
+        const int m_tiles = (g.Mg + 16 * mb - 1) / (16 * mb);
+        const double unit_us = (tpp + 1) / 2 * PAIR_US * (mb == 8 ? (npiece == 2 ? 1.3 : 1.1) : 1.0);
+        for (int ks = 1; ks <= (lean ? 1 : std::min(units, 64)); ++ks) {
+            const int per = (units + ks - 1) / ks;
+            if ((units + per - 1) / per != ks) continue;   // the same units per share with fewer shares
+            if (ks > 1 && out_bytes * ks > (double)SHARE_BYTES_MAX) break;
+            const long long rounds = (spatial * m_tiles * ks + 255) / 256;
+            const double us = rounds * (SHARE_US + per * unit_us) + (ks > 1 ? SUM_US + 2 * ks * out_bytes / SUM_BYTES_PER_US : 0.0);
+            if (best == 0.0 || us < best) {
+                best = us;
+                f.mb = mb;
+                f.ksplit = ks;
+                f.units_per = per;
+            }
+        }
+    }
+}
+}  // namespace
+
+FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, bool lean) {
     FwdWin f{};
     f.ok = false;
     wt = base;
     if (!base.ok || g.Mg < 16) return f;
-    // 128-row tiles unless the GEMM side is small or the grid would leave CUs idle
-    // (one workgroup per CU at a time: the window takes most of the LDS)
+    // 3D samples taps in groups of four: passes of eight taps fill their groups (27 taps:
+    // 8, 8, 8, 3 = seven groups, where passes of nine would take nine)
+    const int tpp = dim == 3 && g.Kn > WIN_TMAX ? 8 : base.tpp;
     const long long spatial = (long long)g.G * g.B * base.ntile[0] * base.ntile[1] * base.ntile[2];
-    f.mb = (dim == 3 || g.Mg <= 64 || spatial * ((g.Mg + 127) / 128) < 256) ? 4 : 8;
-    const int rows = 16 * f.mb;
-    const long long max_cells = (long long)xq_of(f.mb) * NT / 4;
+    const int slices = (g.Cg + BC - 1) / BC;
     // (3D: one more cell, the zero cell)
     const int zc = dim == 3 ? 1 : 0;
-    wt = win_resize(base, g, dim, (size_t)(GEO_WORDS + zc * XS) * sizeof(float), XS * sizeof(float), max_cells - zc);
+    // window of a tile of mb row blocks beside `extra` bytes of LDS (XQ quads prefetched per thread)
+    auto window = [&](int mb, int extra) {
+        return win_resize(base, g, dim, (size_t)(GEO_WORDS + zc * XS) * sizeof(float) + extra, XS * sizeof(float),
+                          (long long)xq_of(mb) * NT / 4 - zc);
+    };
+    // 128-row tiles prefetch fewer window cells: not where that costs the window its margin (strided
+    // layers, whose samples outside it would go to global memory)
+    const bool wide = dim < 3 && g.Mg > 64 && window(8, 0).R[2] >= std::min(window(4, 0).R[2], 4);
+    split_shares(f, g, wide ? 8 : 4, spatial, slices, tpp, base.npiece, lean);
+    const int rows = 16 * f.mb;
+    const long long max_cells = (long long)xq_of(f.mb) * NT / 4;
+    wt = window(f.mb, 0);
     if (wt.cells == 0) return f;   // no window fits: the unwindowed forward
     // 1D / 2D: two staging buffers of the 16-bit loop's weight blocks (8 row blocks x npiece KB
     // each: one step of 128-row tiles or two of 64-row tiles) when the window keeps a margin of
@@ -734,9 +814,7 @@ FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt) {
     f.stage_bytes = 0;
     if (dim < 3) {
         const int stage = 2 * 8 * base.npiece * 1024;
-        const WinTiles ws =
-            win_resize(base, g, dim, (size_t)(GEO_WORDS + zc * XS) * sizeof(float) + stage, XS * sizeof(float),
-                       max_cells - zc);
+        const WinTiles ws = window(f.mb, stage);
         const int e = 2;   // the last axis: used in every rank
         if (ws.cells > 0 && ws.R[e] >= std::min(wt.R[e], 4)) {
             wt = ws;
@@ -748,14 +826,7 @@ FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt) {
     f.m_tiles = (g.Mg + rows - 1) / rows;
     f.Mg_pad = f.m_tiles * rows;
     f.Cg_pad = (g.Cg + BC - 1) / BC * BC;
-    // a grid that cannot give every CU a workgroup splits the channel slices in two (fp32
-    // partials added onto a zeroed output: deterministic for two shares)
-    const int slices = f.Cg_pad / BC;
-    f.ksplit = (spatial * f.m_tiles < 256 && slices >= 2) ? 2 : 1;
-    f.slices_per = (slices + f.ksplit - 1) / f.ksplit;
-    // 3D samples taps in groups of four: passes of eight taps fill their groups (27 taps:
-    // 8, 8, 8, 3 = seven groups, where passes of nine would take nine)
-    if (dim == 3 && g.Kn > WIN_TMAX) wt.tpp = 8;
+    wt.tpp = tpp;
     // 16-bit weight fragments
     f.npiece = base.npiece;
     f.tpp = wt.tpp;
@@ -810,17 +881,44 @@ hipError_t launch_fwd_win_layout16(int dtype, const Geo &g, const FwdWin &fw, co
     return hipErrorInvalidValue;
 }
 
+static hipError_t launch_share_sum(int dtype, const Geo &g, const FwdWin &fw, const void *y32, void *y, hipStream_t s) {
+    const size_t n = (size_t)g.B * g.M * g.Pn;
+    // (the planes start at multiples of n values of an aligned buffer)
+    auto go = [&](auto tv) {
+        using T = decltype(tv);
+        const bool vec = n % 4 == 0 && reinterpret_cast<uintptr_t>(y) % (4 * sizeof(T)) == 0;
+        const size_t items = vec ? n / 4 : n;
+        const dim3 grid((unsigned)((items + 255) / 256));
+        if (vec)
+            hipLaunchKernelGGL((share_sum_kernel<T, true>), grid, dim3(256), 0, s, static_cast<const float *>(y32),
+                               static_cast<T *>(y), n, fw.ksplit);
+        else
+            hipLaunchKernelGGL((share_sum_kernel<T, false>), grid, dim3(256), 0, s, static_cast<const float *>(y32),
+                               static_cast<T *>(y), n, fw.ksplit);
+        return hipGetLastError();
+    };
+    switch (dtype) {
+        case kF32: return go(float());
+        case kF16: return go(__half());
+        case kBF16: return go(__hip_bfloat16());
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl,
                           const void *wf, const void *w16, const int *flag, const void *offset, const void *mask,
                           const void *bias, void *y, void *y32, hipStream_t s) {
     if (fw.ksplit != 1 && y32 == nullptr) return hipErrorInvalidValue;
+    if (g.B == 0) return hipSuccess;
+    hipError_t e = hipErrorInvalidValue;
     switch (dtype) {
-        case kF32: return launch_d<float>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
-        case kF16: return launch_d<__half>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+        case kF32: e = launch_d<float>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s); break;
+        case kF16: e = launch_d<__half>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s); break;
         case kBF16:
-            return launch_d<__hip_bfloat16>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+            e = launch_d<__hip_bfloat16>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+            break;
     }
-    return hipErrorInvalidValue;
+    return e != hipSuccess || fw.ksplit == 1 ? e : launch_share_sum(dtype, g, fw, y32, y, s);
 }
 
 }  // namespace tvdcn_hip

@@ -97,9 +97,9 @@ struct FwdWin {
     bool ok;
     int mb;              // 16-row blocks per workgroup (8 or 4)
     int m_tiles;         // (16 * mb)-row blocks of the GEMM side
-    int ksplit;          // 1, or 2: the channel slices split between two workgroups whose fp32
-                         // partials are added onto a zeroed fp32 output (y32)
-    int slices_per;      // 16-channel slices per share
+    int ksplit;          // shares of the (pass, 16-channel slice) units of a tile: 1, or more, each a
+                         // workgroup storing its fp32 partial to a plane of y32, summed in order
+    int units_per;       // units per share
     int Mg_pad, Cg_pad;  // padded weight layout Wf[G][Kn][Mg_pad][Cg_pad]
     // 16x16x32 MFMAs over (tap pair, 16 channels) steps (1D / 2D): the weight as
     // W16[G][slices][pp][Mg_pad / 16][npiece][512] 16-bit values, pp = passes x hp tap pairs
@@ -110,8 +110,8 @@ struct FwdWin {
 
 FwdTiles plan_fwd(const Geo &g, int dtype);
 // windowed forward plan over the base tiling; wt receives the tiling with the forward's
-// own window margin
-FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt);
+// own window margin (lean: one share per tile, so no partials in the workspace)
+FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, bool lean = false);
 WeightWin plan_weight_win(const Geo &g, const WinTiles &wt, int dim);
 WinTiles plan_data_win(const Geo &g, int dtype, int dim, bool scatter, bool coord);
 // the same tiling with the window margin re-sized for another kernel's LDS budget
@@ -203,7 +203,9 @@ hipError_t launch_fwd_win_layout(int dtype, const Geo &g, const FwdWin &fw, cons
 // (wp: when not null, also the fp32 layout of launch_fwd_win_layout, in the same launch)
 hipError_t launch_fwd_win_layout16(int dtype, const Geo &g, const FwdWin &fw, const void *w, void *w16, int *flag,
                                    hipStream_t s, void *wp = nullptr);
-// w16 / flag: the 16-bit weight and the operand flag (w16 null, or *flag set: the fp32 loop)
+// w16 / flag: the 16-bit weight and the operand flag (w16 null, or *flag set: the fp32 loop);
+// y32: FwdWin::ksplit planes of B * M * Pn floats when there is more than one share (then summed into
+// y by a second launch), else not used
 hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl,
                           const void *wf, const void *w16, const int *flag, const void *offset, const void *mask,
                           const void *bias, void *y, void *y32, hipStream_t s);
