@@ -5,6 +5,7 @@ import ctypes
 import pytest
 import torch
 
+import tvdcn
 from helpers import make_case, rel_err
 from test_gpu_parity import check
 from test_zz_no_alloc import SCRATCH_BYTES, _desc, _lib, _run
@@ -73,3 +74,52 @@ def test_forward_without_room_for_partial_sums():
     assert lib.tvdcn_deform_conv_forward_workspace_size(ctypes.byref(d)) > SCRATCH_BYTES
     y = _run(lib, case, torch.float32, noalloc=True)
     assert rel_err(y, _run(lib, case, torch.float32, noalloc=False)) < 9e-6
+
+
+# few sampled-side channels: column lengths (channels x taps) around the 16 and 64 blocks and at the rule's
+# ends, GEMM sides around 16 and 64, pixels around the 64 of a tile, more tiles than workgroups, offset and
+# mask groups that do not nest, conv groups, no offset / mask / bias
+FEW = [
+    # dim, transposed, make_case arguments
+    (1, False, dict(batch=1, cin=1, cout=1, kernel=[1], in_size=[1])),
+    (1, False, dict(batch=3, cin=2, cout=17, kernel=[8], in_size=[26])),                       # 16 values, 63 pixels
+    (2, False, dict(batch=2, cin=3, cout=65, kernel=[3, 3], in_size=[4, 8])),                  # 27, 64 pixels
+    (2, False, dict(batch=5, cin=13, cout=16, kernel=[5, 1], in_size=[3, 9])),                # 65, 55 pixels
+    (2, False, dict(batch=1, cin=6, cout=10, kernel=[3, 3], in_size=[9, 9], og=2, mg=3, groups=2)),
+    (2, False, dict(batch=2, cin=6, cout=6, kernel=[2, 2], in_size=[5, 13], og=3, mg=1, groups=6, bias=False)),
+    (2, False, dict(batch=9, cin=14, cout=5, kernel=[3, 3], in_size=[45, 44])),                # 126, two tiles a workgroup
+    (3, False, dict(batch=1, cin=5, cout=9, kernel=[3, 3, 4], in_size=[5, 6, 7])),             # 180
+    (2, False, dict(batch=2, cin=3, cout=4, kernel=[3, 3], in_size=[7, 7], deformable=False)),
+    (2, False, dict(batch=2, cin=3, cout=4, kernel=[3, 3], in_size=[7, 7], modulated=False)),
+    (1, False, dict(batch=2, cin=3, cout=4, kernel=[3], in_size=[7], deformable=False, modulated=False)),
+    (2, True, dict(batch=2, cin=66, cout=3, kernel=[4, 4], in_size=[5, 7])),
+    (3, True, dict(batch=1, cin=6, cout=2, kernel=[2, 3, 2], in_size=[3, 4, 5], groups=2, og=2, bias=False)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16, torch.bfloat16],
+                         ids=["f32", "f64", "f16", "bf16"])
+@pytest.mark.parametrize("i", range(len(FEW)))
+def test_few_channels(i, dtype):
+    dim, transposed, kw = FEW[i]
+    stride = 2 if transposed else 1
+    check(make_case(dim, transposed, stride=[stride] * dim, padding=[1] * dim, dilation=[1] * dim, out_pad=[0] * dim,
+                    seed=60 + i, **kw), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_few_channels_last(dtype):
+    """A channels-last input gives the contiguous input's results (the same operations: only the order of the
+    scatter's float atomics differs) and a channels-last gradient."""
+    case = make_case(2, batch=2, cin=5, cout=7, kernel=[3, 3], stride=[1, 1], padding=[1, 1], dilation=[1, 1],
+                     in_size=[9, 11], seed=80)
+    outs = []
+    for fmt in (torch.contiguous_format, torch.channels_last):
+        ts = [case[n].to("cuda", dtype) for n in ("input", "weight", "offset", "mask", "bias")]
+        ts[0] = ts[0].contiguous(memory_format=fmt)
+        ts = [t.requires_grad_(True) for t in ts]
+        y = tvdcn.deform_conv2d(*ts, padding=1)
+        outs.append((y,) + torch.autograd.grad(y.float().square().sum(), ts))
+    assert outs[1][1].is_contiguous(memory_format=torch.channels_last)
+    for a, b in zip(*outs):
+        assert rel_err(a, b) < (1e-6 if dtype == torch.float32 else 1e-2)

@@ -80,6 +80,7 @@ struct Plan {
     WinTiles wn_f;   // the wn_s tiling with the forward kernel's window margin
     WeightWin ww;    // windowed weight-gradient plan (over wn_w)
     FwdWin fw;       // windowed forward plan (over wn_f)
+    FewPlan few;     // layers of few channels that the windowed kernels do not take
     // conv backward: grad_input accumulated in the caller's tensor, no channels-last accumulator
     // (a channels-last input of the accumulation type, or float32 on the windowed data gradient,
     // whose window flush and atomics address the (B, C, *S) tensor directly)
@@ -207,6 +208,8 @@ tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch, bool l
                                x_window_cell_bytes());
     pl.ww = plan_weight_win(g, pl.wn_w, pl.dim);
     pl.fw = plan_fwd_win(g, pl.wn_s, pl.dim, pl.wn_f, lean);
+    pl.few = plan_few(g, pl.dtype);
+    if (pl.wn_s.ok) pl.few.ok = false;
     const bool cl_in = (d->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
     // (1D only: there a window row is the tile's 256 pixels + margins, whole lines of each channel;
     // 2D / 3D window rows are 10-26 cells, and the flush and out-of-window corners then reach
@@ -315,6 +318,13 @@ Layout layout(const Plan &pl, bool backward) {
     L.xcl = L.wf = L.wd = L.cl_acc = L.wpart = L.goff_acc = L.gmask_acc = L.yacc = SENTINEL;
     L.zs = L.wsplit = L.w16 = L.flag = L.zw = SENTINEL;
     L.flag = take(align_up(sizeof(int) * OPERAND_FLAG_WORDS));   // the flag and the operands' largest magnitudes
+    if (pl.few.ok) {
+        // the input gradient / transposed output in the accumulation type, the weight gradient's sums
+        if (!acc_is_storage(pl.dtype) && backward != pl.transposed) L.cl_acc = take(cl_bytes);
+        if (backward) L.wpart = take(align_up(pl.few.part_elems * a));
+        L.total = off;
+        return L;
+    }
     // windowed data gradient (conv backward, transposed forward and backward): split operands
     auto take_split = [&]() {
         if (!pl.wn_s.ok) return;
@@ -547,6 +557,21 @@ tvdcn_status forward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const 
     const int dt = pl.dtype;
     g_last_error.clear();
     int *flag = static_cast<int *>(at(workspace, L.flag));
+    if (pl.few.ok) {
+        const bool cl = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
+        if (!pl.transposed) {
+            TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
+                         launch_few_fwd(dt, pl.dim, g, input, cl, weight, offset, mask, bias, output, s));
+            return TVDCN_STATUS_SUCCESS;
+        }
+        void *y = acc_is_storage(dt) ? output : at(workspace, L.cl_acc);
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_few_init(dt, g, y, bias, s));
+        TVDCN_LAUNCH(TVDCN_KERNEL_DATA_GRAD, s, launch_few_data(dt, pl.dim, g, pl.few, input, nullptr, false, weight, offset,
+                                                                mask, y, nullptr, nullptr, nullptr, s));
+        if (y != output)
+            TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_acc_to_storage(dt, y, output, (size_t)g.B * g.C * g.Sn, s));
+        return TVDCN_STATUS_SUCCESS;
+    }
     if (!pl.transposed) {
         void *xcl = at(workspace, L.xcl), *wf = at(workspace, L.wf);
         void *w16 = pl.fw.ok && sampled16_host_ok(pl, desc) ? at(workspace, L.w16) : nullptr;
@@ -629,7 +654,27 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
     // X: the sampled tensor (conv: input; transposed: grad_out)
     const void *Z = pl.transposed ? input : grad_out;
     const void *X = pl.transposed ? grad_out : input;
-    {
+    if (pl.few.ok) {
+        const bool cl = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
+        void *gx = pl.transposed ? nullptr : direct ? grad_input : at(workspace, L.cl_acc), *part = at(workspace, L.wpart);
+        const size_t n_x = (size_t)g.B * g.C * g.Sn;
+        if (gx != nullptr) {
+            const FillItem fills[1] = {{gx, n_x * ab}};
+            TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 1, s));
+        } else {
+            TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
+                         launch_few_fwd(dt, pl.dim, g, X, cl, weight, offset, mask, nullptr, grad_input, s));
+            TVDCN_LAUNCH(TVDCN_KERNEL_BIAS_GRAD, s,
+                         launch_bias_grad(dt, grad_out, grad_bias, g.B, g.C, g.Sn, s, accumulate_weight));
+        }
+        TVDCN_LAUNCH(TVDCN_KERNEL_DATA_GRAD, s, launch_few_data(dt, pl.dim, g, pl.few, Z, X, cl, weight, offset, mask, gx,
+                                                                grad_offset, grad_mask, part, s));
+        TVDCN_LAUNCH(TVDCN_KERNEL_WEIGHT_GRAD, s, launch_few_reduce(dt, g, pl.few, part, grad_weight,
+                                                                    pl.transposed ? nullptr : grad_bias,
+                                                                    accumulate_weight, s));
+        if (gx != nullptr && !direct)
+            TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_acc_to_storage(dt, gx, grad_input, n_x, s));
+    } else {
         void *xcl = at(workspace, L.xcl), *wd = at(workspace, L.wd);
         int *flag = static_cast<int *>(at(workspace, L.flag));
         const bool cl_in = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;   // conv only
@@ -749,7 +794,7 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
     if (gmask && (desc->flags & TVDCN_FLAG_MASK_SOFTMAX))
         TVDCN_LAUNCH(TVDCN_KERNEL_MASK_SOFTMAX, s,
                      launch_mask_softmax_logit_grad(dt, mask, gmask, (int64_t)g.B * g.mg, g.Kn, g.Pn, s));
-    if (!direct && (goff || gmask))
+    if (!direct && !pl.few.ok && (goff || gmask))
         TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
                      launch_acc_to_storage2(dt, goff, grad_offset, goff ? n_goff : 0, gmask, grad_mask,
                                             gmask ? n_gmask : 0, s));

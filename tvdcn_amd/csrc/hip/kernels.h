@@ -108,7 +108,16 @@ struct FwdWin {
     int stage_bytes;     // LDS past the X window: the 16-bit loop's two weight staging buffers
 };
 
+// Layers of few sampled-side channels (few_channels.hip): the columns of 64-pixel tiles whole in LDS
+struct FewPlan {
+    bool ok;             // a pixel's column, C * Kn values, fits (and any mask activation is finished in fp32 / fp64)
+    int chunks;          // 64-pixel tiles per workgroup of the data kernel
+    int splits;          // its workgroups
+    size_t part_elems;   // accumulator elements of their weight / bias gradient sums: [splits][M][Cg * Kn + 1]
+};
+
 FwdTiles plan_fwd(const Geo &g, int dtype);
+FewPlan plan_few(const Geo &g, int dtype);
 // windowed forward plan over the base tiling; wt receives the tiling with the forward's
 // own window margin (lean: one share per tile, so no partials in the workspace)
 FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, bool lean = false);
@@ -246,6 +255,21 @@ hipError_t launch_weight_reduce(int dtype, const Geo &g, int k_splits, const voi
 hipError_t launch_bwd_weight(int dtype, int dim, const Geo &g, const WeightTiles &t, const void *z, const void *xcl,
                              const void *offset, const void *mask, void *part, void *gw, bool accumulate,
                              hipStream_t s);
+
+// few sampled-side channels (few_channels.hip). x, and gx beside it, in (B, C, *S) order or, x_cl, channels-last.
+// y = bias + W * columns of x (conv forward; transposed: grad_input of grad_out)
+hipError_t launch_few_fwd(int dtype, int dim, const Geo &g, const void *x, bool x_cl, const void *w, const void *offset,
+                          const void *mask, const void *bias, void *y, hipStream_t s);
+// gx (accumulation type, added to; null: none), goff / gmask (storage type, written; null: none; x must be
+// given), part (null: no weight gradient)
+hipError_t launch_few_data(int dtype, int dim, const Geo &g, const FewPlan &f, const void *z, const void *x, bool x_cl,
+                           const void *w, const void *offset, const void *mask, void *gx, void *goff, void *gmask,
+                           void *part, hipStream_t s);
+// gw and gb (null: none) from the data kernel's sums (accumulate: added to them)
+hipError_t launch_few_reduce(int dtype, const Geo &g, const FewPlan &f, const void *part, void *gw, void *gb,
+                             bool accumulate, hipStream_t s);
+// y (accumulation type, (B, C, *S)) = bias[c] (null: 0)
+hipError_t launch_few_init(int dtype, const Geo &g, void *y, const void *bias, hipStream_t s);
 
 // mask_softmax (mask_softmax.hip)
 hipError_t launch_mask_softmax_fwd(int dtype, const void *x, void *y, int64_t BG, int K, int64_t S, hipStream_t s);
