@@ -50,6 +50,10 @@ FORWARD = [
     (1, 33, 32, 300, [257], [3], False),         # 198 tiles of 128 rows
     (3, 1, 40, 16, [4, 9, 9], [3, 3, 3], False),  # four passes of three slices
     (2, 2, 36, 72, [9, 11], [4, 4], True),       # grad_input: two passes of five slices, strided
+    # four pixels per store: rows of the grid in whole quads, boxes four wide, rows past the GEMM side
+    (2, 1, 32, 70, [18, 20], [3, 3], False),
+    (2, 2, 16, 19, [33, 4], [1, 1], False),
+    (1, 40, 16, 260, [300], [1], False),
 ]
 
 

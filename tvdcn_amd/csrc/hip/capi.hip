@@ -337,7 +337,7 @@ Layout layout(const Plan &pl, bool backward) {
     };
     // the fp32 partials of a windowed forward in shares
     const bool split_acc = pl.fw.ok && pl.fw.ksplit > 1;
-    const size_t yacc_bytes = align_up((size_t)pl.fw.ksplit * g.B * g.M * g.Pn * sizeof(float));
+    const size_t yacc_bytes = align_up(pl.fw.part_elems * sizeof(float));
     if (!backward) {
         if (!pl.transposed) {
             L.xcl = take(cl_bytes);

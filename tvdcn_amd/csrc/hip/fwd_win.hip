@@ -41,6 +41,42 @@ static_assert(NW * PB * 16 == BPX, "one tile of pixels per workgroup");
 
 constexpr int GEO_WORDS = TM * BPX * 4;
 
+// lanes 4a .. 4a + 3 hold r[v] of row v at pixels 4a .. 4a + 3: on return lane 4a + i holds row i's four
+// pixels (two exchanges within lane quads)
+__device__ __forceinline__ void transpose_quad(acc4 &r, int lane) {
+    auto swap = [&](auto ctrl, bool hi, int lo_v, int hi_v) {
+        const float send = hi ? r[lo_v] : r[hi_v];
+        const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), decltype(ctrl)::value, 0xF, 0xF, true));
+        r[lo_v] = hi ? got : r[lo_v];
+        r[hi_v] = hi ? r[hi_v] : got;
+    };
+    const std::integral_constant<int, 0xB1> x1;   // lane ^ 1
+    const std::integral_constant<int, 0x4E> x2;   // lane ^ 2
+    swap(x1, lane & 1, 0, 1);
+    swap(x1, lane & 1, 2, 3);
+    swap(x2, lane & 2, 0, 2);
+    swap(x2, lane & 2, 1, 3);
+}
+
+// 16 rows (m0 .. m0 + 15 of the group's rows at yg) x 16 pixels, lane (pixel l % 16 = p, rows 4 (l / 16) ..):
+// vec (P_x % 4 == 0: the lane quad's pixels are consecutive, all inside the grid or all outside, and 4-aligned):
+// one row's four pixels per lane, else four single values
+template <typename T>
+__device__ __forceinline__ void store_frag(const Geo &g, T *yg, int m0, int p, bool vec, acc4 r) {
+    const int lane = threadIdx.x & 63;
+    const int m = m0 + 4 * (lane >> 4);
+    if (vec) {
+        transpose_quad(r, lane);
+        const int mi = m + (lane & 3);
+        if (p >= 0 && mi < g.Mg)
+            store4_t<T, float>(yg + (size_t)mi * g.Pn + (p - (lane & 3)), Vec4<float>{r[0], r[1], r[2], r[3]});
+    } else if (p >= 0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (m + v < g.Mg) yg[(size_t)(m + v) * g.Pn + p] = from_acc<T, float>(r[v]);
+    }
+}
+
 // STAGE: the 16-bit loop's weight blocks are staged in LDS (1D / 2D, fw.stage_bytes > 0)
 template <int DIM, typename T, int MB, bool STAGE>
 __global__ void __launch_bounds__(NT)
@@ -579,51 +615,60 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
         }
     }
 
-    // ---- epilogue: + bias, store NC<spatial>. With several shares each stores its fp32 partial
-    //      to its own plane of y32 (bias with the first share); share_sum_kernel adds the planes in
-    //      order, so the result is deterministic.
+    // ---- epilogue: + bias, store NC<spatial>. With several shares each stores its fp32 partial to
+    //      its own plane of y32 in the accumulators' order (whole 1 KB wave stores; in y's order the
+    //      partials of 128 rows x 256 pixels took half of a one-slice workgroup's 36 us), bias with
+    //      the first share; share_sum_kernel adds the planes in order, so the result is deterministic.
+    const size_t tile_id = ((size_t)grp * n_sp + sp) * fw.m_tiles + mt;
+    float *frag = nullptr;
+    if (fw.ksplit > 1)
+        frag = y32 + ((((size_t)ks * g.G * n_sp * fw.m_tiles + tile_id) * NW + wave) * (MB * PB)) * 256 + lane * 4;
+    int pix[PB];
 #pragma unroll
-    for (int pb = 0; pb < PB; ++pb) {
-        const int p = tile.pixel(g, wt, wave * (PB * 16) + pb * 16 + (lane & 15));
-        if (p < 0) continue;
+    for (int pb = 0; pb < PB; ++pb) pix[pb] = tile.pixel(g, wt, wave * (PB * 16) + pb * 16 + (lane & 15));
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < MB; ++mb) {
+        const int m0 = mt * BMR + mb * 16;
+        acc4 bv = acc4{0.f, 0.f, 0.f, 0.f};
+        if (bias != nullptr && ks == 0)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = mt * BMR + mb * 16 + 4 * q + v;
-                if (m < g.Mg) {
-                    const int mg_glob = grp * g.Mg + m;
-                    float r = s_back != 0 ? ldexpf(acc[mb][pb][v], s_back) : acc[mb][pb][v];
-                    if (bias != nullptr && ks == 0) r += to_acc<float>(bias[mg_glob]);
-                    const size_t o = ((size_t)tile.b * g.M + mg_glob) * g.Pn + p;
-                    if (fw.ksplit == 1)
-                        y[o] = from_acc<T, float>(r);
-                    else
-                        y32[(size_t)ks * g.B * g.M * g.Pn + o] = r;
-                }
-            }
+            for (int v = 0; v < 4; ++v) bv[v] = to_acc<float>(bias[grp * g.Mg + min(m0 + 4 * q + v, g.Mg - 1)]);
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            acc4 r = acc[mb][pb];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) r[v] = (s_back != 0 ? ldexpf(r[v], s_back) : r[v]) + bv[v];
+            if (fw.ksplit > 1)
+                *reinterpret_cast<acc4 *>(frag + (mb * PB + pb) * 256) = r;
+            else
+                store_frag<T>(g, y + ((size_t)tile.b * g.M + (size_t)grp * g.Mg) * g.Pn, m0, pix[pb], fw.vec, r);
+        }
     }
 }
 
-// y[i] = sum over the shares k of part[k][i], in order (n values per share). VEC: 16-byte loads
-// (n % 4 == 0). Bound by the partials' bytes, read once each.
-template <typename T, bool VEC>
-__global__ void __launch_bounds__(256) share_sum_kernel(const float *__restrict__ part, T *__restrict__ y, size_t n,
-                                                        int shares) {
-    constexpr int W = VEC ? 4 : 1;
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * W;
-    if (i >= n) return;
-    if constexpr (VEC) {
-        acc4 v = *reinterpret_cast<const acc4 *>(part + i);
+// The fragments of share_sum: wave = 16 rows x 16 pixels of one tile, summed over the shares in order and
+// stored in y's order. Bound by the partials' bytes, read once each.
+template <typename T, int MB>
+__global__ void __launch_bounds__(256) share_sum_kernel(const Geo g, const WinTiles wt, const FwdWin fw,
+                                                        const float *__restrict__ part, T *__restrict__ y, size_t frags) {
+    const int lane = threadIdx.x & 63;
+    const size_t f = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // ((tile * NW + wave) * MB + mb) * PB + pb
+    if (f >= frags) return;
+    const float *src = part + f * 256 + lane * 4;
+    acc4 v = *reinterpret_cast<const acc4 *>(src);
 #pragma unroll 4
-        for (int k = 1; k < shares; ++k) v += *reinterpret_cast<const acc4 *>(part + (size_t)k * n + i);
-        store4_t<T, float>(y + i, Vec4<float>{v[0], v[1], v[2], v[3]});
-    } else {
-        float v = part[i];
-#pragma unroll 4
-        for (int k = 1; k < shares; ++k) v += part[(size_t)k * n + i];
-        y[i] = from_acc<T, float>(v);
-    }
+    for (int k = 1; k < fw.ksplit; ++k) v += *reinterpret_cast<const acc4 *>(src + (size_t)k * frags * 256);
+    const int i = (int)(f % (NW * MB * PB));
+    const int pb = i % PB, mb = i / PB % MB, wave = i / (PB * MB);
+    int L = (int)(f / (NW * MB * PB));
+    const int mt = L % fw.m_tiles;
+    L /= fw.m_tiles;
+    const int n_sp = g.B * wt.ntile[0] * wt.ntile[1] * wt.ntile[2];
+    const int grp = L / n_sp;
+    Tile tile;
+    tile.init(g, wt, L % n_sp, 0, grp);
+    store_frag<T>(g, y + ((size_t)tile.b * g.M + (size_t)grp * g.Mg) * g.Pn, (mt * MB + mb) * 16,
+                  tile.pixel(g, wt, wave * (PB * 16) + pb * 16 + (lane & 15)), fw.vec, v);
 }
 
 // weight (M, Cg, Kn) -> Wp[G][slices][Kn][Mg_pad / 16][16 m][16 c], zero padded (grid-stride loop
@@ -761,10 +806,10 @@ constexpr double SHARE_US = 8.0, PAIR_US = 2.0, SUM_US = 5.0, SUM_BYTES_PER_US =
 constexpr size_t SHARE_BYTES_MAX = (size_t)64 << 20;   // partials of one call
 void split_shares(FwdWin &f, const Geo &g, int mb_max, long long spatial, int slices, int tpp, int npiece, bool lean) {
     const int npass = (g.Kn + tpp - 1) / tpp, units = npass * slices;
-    const double out_bytes = 4.0 * g.B * g.M * g.Pn;
     double best = 0.0;
     for (int mb = mb_max; mb >= 4; mb -= 4) {
         const int m_tiles = (g.Mg + 16 * mb - 1) / (16 * mb);
+        const double out_bytes = 4.0 * spatial * m_tiles * (16 * mb * BPX);   // a share's partials
         const double unit_us = (tpp + 1) / 2 * PAIR_US * (mb == 8 ? (npiece == 2 ? 1.3 : 1.1) : 1.0);
         for (int ks = 1; ks <= (lean ? 1 : std::min(units, 64)); ++ks) {
             const int per = (units + ks - 1) / ks;
@@ -827,6 +872,8 @@ FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, b
     f.Mg_pad = f.m_tiles * rows;
     f.Cg_pad = (g.Cg + BC - 1) / BC * BC;
     wt.tpp = tpp;
+    f.part_elems = f.ksplit > 1 ? (size_t)f.ksplit * spatial * f.m_tiles * rows * BPX : 0;
+    f.vec = g.P[2] % 4 == 0 && wt.box[2] % 4 == 0;
     // 16-bit weight fragments
     f.npiece = base.npiece;
     f.tpp = wt.tpp;
@@ -881,35 +928,36 @@ hipError_t launch_fwd_win_layout16(int dtype, const Geo &g, const FwdWin &fw, co
     return hipErrorInvalidValue;
 }
 
-static hipError_t launch_share_sum(int dtype, const Geo &g, const FwdWin &fw, const void *y32, void *y, hipStream_t s) {
-    const size_t n = (size_t)g.B * g.M * g.Pn;
-    // (the planes start at multiples of n values of an aligned buffer)
-    auto go = [&](auto tv) {
+static hipError_t launch_share_sum(int dtype, const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *y32, void *y,
+                                   hipStream_t s) {
+    const size_t frags = fw.part_elems / fw.ksplit / 256;
+    const dim3 grid((unsigned)((frags + 3) / 4));
+    auto go = [&](auto tv, auto mv) {
         using T = decltype(tv);
-        const bool vec = n % 4 == 0 && reinterpret_cast<uintptr_t>(y) % (4 * sizeof(T)) == 0;
-        const size_t items = vec ? n / 4 : n;
-        const dim3 grid((unsigned)((items + 255) / 256));
-        if (vec)
-            hipLaunchKernelGGL((share_sum_kernel<T, true>), grid, dim3(256), 0, s, static_cast<const float *>(y32),
-                               static_cast<T *>(y), n, fw.ksplit);
-        else
-            hipLaunchKernelGGL((share_sum_kernel<T, false>), grid, dim3(256), 0, s, static_cast<const float *>(y32),
-                               static_cast<T *>(y), n, fw.ksplit);
+        hipLaunchKernelGGL((share_sum_kernel<T, decltype(mv)::value>), grid, dim3(256), 0, s, g, wt, fw,
+                           static_cast<const float *>(y32), static_cast<T *>(y), frags);
         return hipGetLastError();
     };
+    auto by_mb = [&](auto tv) {
+        return fw.mb == 8 ? go(tv, std::integral_constant<int, 8>()) : go(tv, std::integral_constant<int, 4>());
+    };
     switch (dtype) {
-        case kF32: return go(float());
-        case kF16: return go(__half());
-        case kBF16: return go(__hip_bfloat16());
+        case kF32: return by_mb(float());
+        case kF16: return by_mb(__half());
+        case kBF16: return by_mb(__hip_bfloat16());
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl,
+hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw_, const void *xcl,
                           const void *wf, const void *w16, const int *flag, const void *offset, const void *mask,
                           const void *bias, void *y, void *y32, hipStream_t s) {
-    if (fw.ksplit != 1 && y32 == nullptr) return hipErrorInvalidValue;
+    if (fw_.ksplit != 1 && y32 == nullptr) return hipErrorInvalidValue;
     if (g.B == 0) return hipSuccess;
+    // (a batch block's output may be less aligned than the caller's)
+    const size_t quad = 4 * (dtype == kF32 ? sizeof(float) : sizeof(uint16_t));
+    FwdWin fw = fw_;
+    fw.vec = fw.vec && reinterpret_cast<uintptr_t>(y) % quad == 0;
     hipError_t e = hipErrorInvalidValue;
     switch (dtype) {
         case kF32: e = launch_d<float>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s); break;
@@ -918,7 +966,7 @@ hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, 
             e = launch_d<__hip_bfloat16>(dim, g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
             break;
     }
-    return e != hipSuccess || fw.ksplit == 1 ? e : launch_share_sum(dtype, g, fw, y32, y, s);
+    return e != hipSuccess || fw.ksplit == 1 ? e : launch_share_sum(dtype, g, wt, fw, y32, y, s);
 }
 
 }  // namespace tvdcn_hip

@@ -100,6 +100,8 @@ struct FwdWin {
     int ksplit;          // shares of the (pass, 16-channel slice) units of a tile: 1, or more, each a
                          // workgroup storing its fp32 partial to a plane of y32, summed in order
     int units_per;       // units per share
+    size_t part_elems;   // floats of the shares' partials (0: one share)
+    bool vec;            // 4 consecutive pixels of a tile row are contiguous and 4-aligned in the output
     int Mg_pad, Cg_pad;  // padded weight layout Wf[G][Kn][Mg_pad][Cg_pad]
     // 16x16x32 MFMAs over (tap pair, 16 channels) steps (1D / 2D): the weight as
     // W16[G][slices][pp][Mg_pad / 16][npiece][512] 16-bit values, pp = passes x hp tap pairs
@@ -213,8 +215,8 @@ hipError_t launch_fwd_win_layout(int dtype, const Geo &g, const FwdWin &fw, cons
 hipError_t launch_fwd_win_layout16(int dtype, const Geo &g, const FwdWin &fw, const void *w, void *w16, int *flag,
                                    hipStream_t s, void *wp = nullptr);
 // w16 / flag: the 16-bit weight and the operand flag (w16 null, or *flag set: the fp32 loop);
-// y32: FwdWin::ksplit planes of B * M * Pn floats when there is more than one share (then summed into
-// y by a second launch), else not used
+// y32: FwdWin::part_elems floats when there is more than one share (their sum is brought into y by a second
+// launch), else not used
 hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl,
                           const void *wf, const void *w16, const int *flag, const void *offset, const void *mask,
                           const void *bias, void *y, void *y32, hipStream_t s);
