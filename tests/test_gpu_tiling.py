@@ -80,6 +80,20 @@ def test_forward_without_room_for_partial_sums():
     assert rel_err(y, _run(lib, case, torch.float32, noalloc=False)) < 9e-6
 
 
+# the 16-bit types' layouts: rows in eights, in fours and odd, channels past a 64-wide copy tile, rows and
+# positions past their tiles, batches, both directions
+HALF_LAYOUTS = [(1, [64], False), (1, [68], False), (1, [67], False), (2, [9, 24], False), (2, [7, 12], True),
+                (3, [3, 4, 8], False), (1, [130], True)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", HALF_LAYOUTS, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
+def test_half_layouts(case, dtype):
+    dim, size, transposed = case
+    check(make_case(dim, transposed, batch=3, cin=68, cout=72, kernel=[3] * dim, stride=[1 + transposed] * dim,
+                    padding=[1] * dim, dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=90 + dim), dtype)
+
+
 # few sampled-side channels: column lengths (channels x taps) around the 16 and 64 blocks and at the rule's
 # ends, GEMM sides around 16 and 64, pixels around the 64 of a tile, more tiles than workgroups, offset and
 # mask groups that do not nest, conv groups, no offset / mask / bias

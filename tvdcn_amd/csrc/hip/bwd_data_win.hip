@@ -57,7 +57,7 @@
 //   * The window (sampled-grid box around the tile's undeformed footprint plus a
 //     margin R per axis) is flushed at the end: one float atomic per non-zero
 //     (cell, channel), 16 consecutive channels per cell.
-#include "window.h"
+#include "operands.h"
 
 namespace tvdcn_hip {
 namespace {
@@ -128,84 +128,6 @@ __device__ __forceinline__ float row_sum4(float v) {
     v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
     const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
-}
-
-// Z (B, G * Mg, Pn) -> zs [B][G][ms32][NP][Pn][32]: per 32-channel step and piece, every pixel's
-// 32 channels (zero past Mg) as 4 lane groups of 8 (the 16x16x32 B-operand layout), so that a
-// wave's fragment load of one piece for 16 consecutive pixels reads 1 KB of whole lines.
-// Block = 64 pixels of one (image, group, step), transposed through LDS.
-// (zvec: Pn % 4 == 0 and z aligned to 4 elements: the tile is read in 4-pixel vectors)
-template <typename T, int NP>
-__device__ __forceinline__ void z_split_block(long long bid, float *smem, const T *__restrict__ z,
-                                              uint16_t *__restrict__ zs, uint16_t *__restrict__ zw, int *flag, int G,
-                                              int Mg, int Pn, int ms32, int pblocks, bool zvec, size_t zw_plane) {
-    float(*tile)[65] = reinterpret_cast<float(*)[65]>(smem);   // [32][65]
-    const int sz = NP == 2 ? operand_scale(flag, AMAX_Z) : 0;   // (every lane: before any returns)
-    // (the block index is a grid index: 32-bit division, not the 64-bit sequence)
-    const unsigned ub = (unsigned)bid;
-    const int pb = (int)(ub % (unsigned)pblocks);
-    const unsigned bgs = ub / (unsigned)pblocks;   // (b * G + grp) * ms32 + step
-    const int st = (int)(bgs % (unsigned)ms32);
-    const unsigned bg = bgs / (unsigned)ms32;
-    const int grp = (int)(bg % (unsigned)G);
-    const unsigned b = bg / (unsigned)G;
-    const int p0 = pb * 64;
-    const T *src = z + ((size_t)b * G + grp) * (size_t)Mg * Pn;
-    if (zvec) {
-        for (int i = threadIdx.x; i < 32 * 16; i += 256) {
-            const int ml = i >> 4, pl = 4 * (i & 15);
-            const int m = st * 32 + ml, p = p0 + pl;
-            Vec4<float> v{0.f, 0.f, 0.f, 0.f};
-            if (m < Mg && p < Pn) v = load4_t<float, T>(src + (size_t)m * Pn + p);   // all four inside
-            tile[ml][pl] = v.x;
-            tile[ml][pl + 1] = v.y;
-            tile[ml][pl + 2] = v.z;
-            tile[ml][pl + 3] = v.w;
-        }
-    } else {
-        for (int i = threadIdx.x; i < 32 * 64; i += 256) {
-            const int ml = i >> 6, pl = i & 63;
-            const int m = st * 32 + ml, p = p0 + pl;
-            float v = 0.f;
-            if (m < Mg && p < Pn) v = to_acc<float>(src[(size_t)m * Pn + p]);
-            tile[ml][pl] = v;
-        }
-    }
-    __syncthreads();
-    if (zw != nullptr) {
-        // the same values for the weight gradient, in 8-pixel column blocks: element (image b, row
-        // m of Z's M, pixel p) at ((b * Pn / 8 + p / 8) * M + m) * 8 + p % 8 of each piece's plane
-        // (Pn % 8 == 0), so that a wave's A fragment (16 rows x 4 blocks of 8 pixels) reads whole
-        // lines. Thread = (row ml, 8-pixel block px / 8): consecutive threads, consecutive rows.
-        const int ml = threadIdx.x & 31, px = 8 * (threadIdx.x >> 5);
-        const int m = st * 32 + ml, pw = p0 + px;
-        if (m < Mg && pw < Pn) {
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = tile[ml][px + e];
-            uint4 out[NP];
-            pack8_16<T, NP>(v, sz, out);
-            const size_t M = (size_t)G * Mg;
-            uint16_t *dst = zw + ((size_t)b * (Pn / 8) + pw / 8) * M * 8 + ((size_t)grp * Mg + m) * 8;
-#pragma unroll
-            for (int k = 0; k < NP; ++k) *reinterpret_cast<uint4 *>(dst + k * zw_plane) = out[k];
-        }
-    }
-    const int pl = threadIdx.x >> 2, q = threadIdx.x & 3, p = p0 + pl;
-    if (p >= Pn) return;
-    float v[8];
-    bool bad = false;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        v[e] = tile[q * 8 + e][pl];
-        bad = bad || split_bad(v[e]);
-    }
-    uint4 out[NP];
-    pack8_16<T, NP>(v, sz, out);
-    uint16_t *dst = zs + ((size_t)bgs * NP * Pn + p) * 32 + q * 8;
-#pragma unroll
-    for (int k = 0; k < NP; ++k) *reinterpret_cast<uint4 *>(dst + (size_t)k * Pn * 32) = out[k];
-    if (NP == 2 && bad) atomicOr(flag, 1);
 }
 
 // Reduction over each row of 16 lanes (the lanes of one channel quad's 16 pixels), the
@@ -281,7 +203,8 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     const int b = tile.b, grp = tile.grp, c0 = tile.c0, cg0 = tile.cg0, ogu = tile.ogu, mgu = tile.mgu;
     const bool deformable = offset != nullptr;
     // the 16-bit K loop when its operands were laid out, and (fp32) none was flagged
-    const int use16_flag = zs != nullptr && (flag == nullptr || *flag == 0);
+    // (fp16 / bf16: always)
+    const int use16_flag = npiece_of<T>() == 1 || (zs != nullptr && (flag == nullptr || *flag == 0));
     const bool cq_ok = c0 + mq < g.Cg;           // Cg % 4 == 0: a channel quad is all in or all out
     const float *xb = xcl + (size_t)b * g.Sn * g.C + cg0;
     // grad_input's strides per channel and per pixel: channels-last (B, S, C) or, gx_nchw, the
@@ -644,7 +567,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         // the whole pass loop)
         int use16 = __builtin_amdgcn_readfirstlane(use16_flag);
         asm volatile("" : "+s"(use16));
-        if (use16) {
+        if (npiece_of<T>() == 1 || use16) {
             if (DIM < 3 && wt.wstage > 0)   // (3D plans stage no weights)
                 kloop16s();
             else if constexpr (NW == 16 && npiece_of<T>() == 1)
@@ -1231,7 +1154,6 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
 // Block = (group, channel slice, row step, run of up to WL_TK taps): reads 16 rows of
 // 16 channels x the run's taps (contiguous runs of taps per channel), transposes through
 // LDS, writes its 256 * taps contiguous output floats.
-constexpr int WL_TK = 8;   // (LDS of the merged layout kernel: 17 KB per block)
 template <typename T>
 __device__ __forceinline__ void weight_win_block(int L, float *smem, const T *__restrict__ w, float *__restrict__ out,
                                                  int G, int Mg, int Cg, int Kn, int c_tiles, int m_steps) {
@@ -1256,52 +1178,6 @@ __device__ __forceinline__ void weight_win_block(int L, float *smem, const T *__
     __syncthreads();
     float *dst = out + ((((size_t)grp * c_tiles + ct) * m_steps + ms) * Kn + t0) * (BC * BM);
     for (int e = threadIdx.x; e < n; e += blockDim.x) dst[e] = tile[e / (BM * BC)][(e / BM) % BC][e % BM];
-}
-
-// weight (M, Cg, Kn) -> split chunks [G][c_tiles][ms32][Kn][NP][4 q][16 c][8 e]: per (step, tap)
-// and piece, the 16x16x32 A-operand fragment of 16 channels x 32 GEMM-side channels (lane
-// q * 16 + c holds rows 8q .. 8q + 7 of channel c; zero past Mg / Cg). Block = (group, channel
-// slice, step, run of up to WL_TK taps), transposed through LDS.
-template <typename T, int NP>
-__device__ __forceinline__ void weight_split_block(int L, float *smem, const T *__restrict__ w,
-                                                   uint16_t *__restrict__ out, int *flag, int G, int Mg, int Cg,
-                                                   int Kn, int c_tiles, int ms32) {
-    float(*tile)[BC][33] = reinterpret_cast<float(*)[BC][33]>(smem);   // [tap][c][m]
-    const int tchunks = (Kn + WL_TK - 1) / WL_TK;
-    const int tc = L % tchunks;
-    L /= tchunks;
-    const int st = L % ms32;
-    L /= ms32;
-    const int ct = L % c_tiles;
-    const int grp = L / c_tiles;
-    const int t0 = tc * WL_TK, nt = min(WL_TK, Kn - t0);
-    const int n = 32 * BC * nt;
-    for (int e = threadIdx.x; e < n; e += blockDim.x) {
-        const int tt = e % nt, r = e / nt;   // (m, c, tap), taps fastest
-        const int ci = r % BC, mi = r / BC;
-        const int m = st * 32 + mi, c = ct * BC + ci;
-        float v = 0.f;
-        if (m < Mg && c < Cg) v = to_acc<float>(w[(((size_t)grp * Mg + m) * Cg + c) * Kn + t0 + tt]);
-        tile[tt][ci][mi] = v;
-    }
-    __syncthreads();
-    uint16_t *dst = out + ((((size_t)grp * c_tiles + ct) * ms32 + st) * Kn + t0) * (NP * 512);
-    const int sw = NP == 2 ? operand_scale(flag, AMAX_W) : 0;
-    bool bad = false;
-    for (int u = threadIdx.x; u < nt * 64; u += blockDim.x) {
-        const int tt = u >> 6, l = u & 63, q = l >> 4, c = l & 15;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            v[e] = tile[tt][c][q * 8 + e];
-            bad = bad || split_bad(v[e]);
-        }
-        uint4 o[NP];
-        pack8_16<T, NP>(v, sw, o);
-#pragma unroll
-        for (int k = 0; k < NP; ++k) *reinterpret_cast<uint4 *>(dst + (size_t)tt * (NP * 512) + k * 512 + l * 8) = o[k];
-    }
-    if (NP == 2 && bad) atomicOr(flag, 1);
 }
 
 // The data gradient's operand layouts in one launch: blocks [0, nz) split Z (z_split_block),
@@ -1565,9 +1441,7 @@ WinTiles plan_data_win(const Geo &g, int dtype, int dim, bool scatter, bool coor
 hipError_t launch_data_win_prep(int dtype, const Geo &g, const WinTiles &t, const void *z, const void *w, void *zs,
                                 void *wsplit, void *wd, int *flag, hipStream_t s, void *zw) {
     switch (dtype) {
-        case kF32: return launch_prep<float>(g, t, z, w, zs, wsplit, wd, flag, s, zw);
-        case kF16: return launch_prep<__half>(g, t, z, w, zs, wsplit, wd, flag, s, zw);
-        case kBF16: return launch_prep<__hip_bfloat16>(g, t, z, w, zs, wsplit, wd, flag, s, zw);
+        case kF32: return launch_prep<float>(g, t, z, w, zs, wsplit, wd, flag, s, zw);   // (fp16 / bf16: launch_prep16)
     }
     return hipErrorInvalidValue;
 }
@@ -1576,6 +1450,7 @@ hipError_t launch_bwd_data_win(int dtype, int dim, const Geo &g, const WinTiles 
                                const void *z, const void *wchunks, const void *zs, const void *wsplit,
                                const int *flag, const void *xcl, const void *offset, const void *mask, void *gx_cl,
                                void *goff, void *gmask, hipStream_t s, bool gx_nchw) {
+    if (dtype != kF32 && (zs == nullptr || wsplit == nullptr)) return hipErrorInvalidValue;
     switch (dtype) {
         case kF32:
             return launch_d<float>(dim, g, t, scatter, coord, z, wchunks, zs, wsplit, flag, xcl, offset, mask, gx_cl,

@@ -302,10 +302,12 @@ Layout layout(const Plan &pl, bool backward) {
     const size_t a = acc_size(pl.dtype);
     const size_t cl_bytes = align_up((size_t)g.B * g.Sn * g.C * a);
     // forward weight layout Wf[G][Kn][Mg_pad][Cg_pad], padded for whichever forward kernel runs
-    const size_t wf_bytes = pl.fw.ok ? align_up((size_t)g.G * g.Kn * pl.fw.Mg_pad * pl.fw.Cg_pad * sizeof(float))
+    // (the windowed kernels' 16-bit types need none of the fp32 loops' layouts)
+    const bool h16 = pl.dtype == kF16 || pl.dtype == kBF16;
+    const size_t wf_bytes = pl.fw.ok && h16 ? 0 : pl.fw.ok ? align_up((size_t)g.G * g.Kn * pl.fw.Mg_pad * pl.fw.Cg_pad * sizeof(float))
                                      : align_up((size_t)g.G * g.Kn * pl.ft.Mg_pad * pl.ft.Cg_pad * a);
     // data-gradient weight: windowed-kernel chunks when eligible, else the [G][Kn][Cg][Mg] layout
-    const size_t wd_bytes = pl.wn_s.ok ? align_up(pl.wn_s.chunk_elems * sizeof(float))
+    const size_t wd_bytes = pl.wn_s.ok && h16 ? 0 : pl.wn_s.ok ? align_up(pl.wn_s.chunk_elems * sizeof(float))
                                        : align_up((size_t)g.G * g.Kn * pl.dt.Mg_pad * pl.dt.Cg_pad * a);
     Layout L;
     size_t off = 0;
@@ -572,7 +574,42 @@ tvdcn_status forward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const 
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_acc_to_storage(dt, y, output, (size_t)g.B * g.C * g.Sn, s));
         return TVDCN_STATUS_SUCCESS;
     }
-    if (!pl.transposed) {
+    const bool h16 = dt == kF16 || dt == kBF16;
+    if (h16 && !pl.transposed && pl.fw.ok) {
+        Prep16 j{};
+        j.x = input;
+        j.x_cl = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
+        j.xcl = at(workspace, L.xcl);
+        j.w = weight;
+        j.w16 = at(workspace, L.w16);
+        j.fw = &pl.fw;
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_prep16(dt, g, j, s));
+        TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
+                     launch_fwd_win(dt, pl.dim, g, pl.wn_f, pl.fw, j.xcl, nullptr, j.w16, nullptr, offset, mask, bias,
+                                    output, at(workspace, L.yacc), s));
+    } else if (h16 && pl.transposed && pl.wn_s.ok) {
+        void *ycl = at(workspace, L.cl_acc);
+        Prep16 j{};
+        j.z = input;
+        j.w = weight;
+        j.zs = at(workspace, L.zs);
+        j.wsplit = at(workspace, L.wsplit);
+        j.wt = &pl.wn_s;
+        j.fill[0] = ycl;
+        j.fill_n[0] = (size_t)g.B * g.Sn * g.C;
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_prep16(dt, g, j, s));
+        TVDCN_LAUNCH(TVDCN_KERNEL_DATA_GRAD, s, launch_bwd_data_win(dt, pl.dim, g, pl.wn_x, true, false, input, nullptr, j.zs,
+                                                                    j.wsplit, nullptr, nullptr, offset, mask, ycl, nullptr,
+                                                                    nullptr, s));
+        Out16 o{};
+        o.acc = ycl;
+        o.y = output;
+        o.bias = bias;
+        o.B = g.B;
+        o.C = g.C;
+        o.S = g.Sn;
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_out16(dt, o, s));
+    } else if (!pl.transposed) {
         void *xcl = at(workspace, L.xcl), *wf = at(workspace, L.wf);
         void *w16 = pl.fw.ok && sampled16_host_ok(pl, desc) ? at(workspace, L.w16) : nullptr;
         const FillItem fills[1] = {{flag, 4 * OPERAND_FLAG_WORDS}};
@@ -675,6 +712,7 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         if (gx != nullptr && !direct)
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_acc_to_storage(dt, gx, grad_input, n_x, s));
     } else {
+        const bool h16 = (dt == kF16 || dt == kBF16) && pl.wn_s.ok;   // the layouts in one launch
         void *xcl = at(workspace, L.xcl), *wd = at(workspace, L.wd);
         int *flag = static_cast<int *>(at(workspace, L.flag));
         const bool cl_in = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;   // conv only
@@ -683,11 +721,40 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         void *gx_cl = pl.transposed ? nullptr : pl.gx_in_place ? grad_input : at(workspace, L.cl_acc);
         // the offset / mask gradient accumulators, the operand flag and grad_input (conv) zeroed by one
         // launch
+        if (h16) {
+            Prep16 j{};
+            j.x = X;
+            j.x_cl = cl_in;
+            j.xcl = xcl;
+            j.z = Z;
+            j.w = weight;
+            j.zs = at(workspace, L.zs);
+            j.wsplit = at(workspace, L.wsplit);
+            j.zw = at(workspace, L.zw);
+            j.wt = &pl.wn_s;
+            if (pl.transposed && pl.fw.ok) {
+                j.w16 = at(workspace, L.w16);
+                j.fw = &pl.fw;
+            }
+            j.gout = grad_out;
+            j.gb = grad_bias;
+            j.bias_c = pl.transposed ? g.C : g.M;
+            j.bias_s = pl.transposed ? g.Sn : g.Pn;
+            j.accumulate = accumulate_weight;
+            j.fill[0] = goff;
+            j.fill_n[0] = n_goff;
+            j.fill[1] = gmask;
+            j.fill_n[1] = n_gmask;
+            j.fill[2] = gx_cl;
+            j.fill_n[2] = (size_t)g.B * g.Sn * g.C;
+            TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_prep16(dt, g, j, s));
+            flag = nullptr;
+        }
         const FillItem fills[4] = {{goff, goff ? n_goff * ab : 0},
                                    {gmask, gmask ? n_gmask * ab : 0},
                                    {flag, 4 * OPERAND_FLAG_WORDS},
                                    {gx_cl, gx_cl ? (size_t)g.B * g.Sn * g.C * ab : 0}};
-        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 4, s));
+        if (!h16) TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fill_zero_multi(fills, 4, s));
         const bool coord = offset != nullptr || mask != nullptr;
         // the 16-bit loops of the sampled side (weight gradient; transposed: input gradient)
         const bool sampled16 = sampled16_host_ok(pl, desc) && (pl.ww.ok || (pl.transposed && pl.fw.ok));
@@ -695,13 +762,13 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         // (fp32) the 16-bit MFMA operands' largest magnitudes: the weight and X ride on X's layout
         // copy, Z = grad_out on the bias gradient (this block's, accumulated over the blocks),
         // whatever else on a launch of its own
-        if (!cl_in) {
+        if (!h16 && !cl_in) {
             // the mask's range check rides on the layout copy
             const void *mchk = sampled16 ? mask_to_check(pl, desc, mask) : nullptr;
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_to_channels_last(dt, X, xcl, g.B, g.C, g.Sn, s, flag, mchk,
                                                                          mask_numel(g), MASK_LIMIT, weight,
                                                                          (size_t)g.M * g.Cg * g.Kn));
-        } else {
+        } else if (!h16) {
             if (direct)
                 x_in_place = xcl = const_cast<void *>(X);   // already the kernels' layout and type
             else
@@ -710,10 +777,10 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         }
         // grad_out (B, Cout, *out_size): conv Cout = M on the column grid, transposed Cout = C on the
         // sampled grid
-        if (!pl.transposed)
+        if (!h16 && !pl.transposed)
             TVDCN_LAUNCH(TVDCN_KERNEL_BIAS_GRAD, s, launch_bias_grad(dt, grad_out, grad_bias, g.B, g.M, g.Pn, s,
                                                                      accumulate_weight, flag));
-        else
+        else if (!h16)
             TVDCN_LAUNCH(TVDCN_KERNEL_BIAS_GRAD, s, launch_bias_grad(dt, grad_out, grad_bias, g.B, g.C, g.Sn, s,
                                                                      accumulate_weight));
         TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, operand_amax(pl, desc, cl_in ? weight : nullptr, cl_in ? X : nullptr,
@@ -722,10 +789,10 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         void *zs = at(workspace, L.zs), *wsp = at(workspace, L.wsplit);
         // (16-bit weight-gradient loop) Z's 16-bit values in column blocks, from the same launch
         void *zw = sampled16 && pl.wn_s.ok ? at(workspace, L.zw) : nullptr;
-        if (pl.wn_s.ok)
+        if (!h16 && pl.wn_s.ok)
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
                          launch_data_win_prep(dt, g, pl.wn_s, Z, weight, zs, wsp, wd, flag, s, zw));
-        else
+        else if (!h16)
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_weight_data_layout(dt, g, weight, wd, pl.dt.Mg_pad, pl.dt.Cg_pad, s));
         if (!pl.transposed) {
             if (pl.wn_s.ok && coord && pl.data_split && pl.dim == 3) {
@@ -748,19 +815,20 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
             else
                 TVDCN_LAUNCH(TVDCN_KERNEL_DATA_GRAD, s, launch_bwd_data(dt, pl.dim, g, pl.dt, true, coord, Z, wd, xcl, offset, mask,
                                                                         gx_cl, goff, gmask, s));
-            if (!pl.gx_in_place && !cl_in)
+            // (h16: with the offset / mask gradients, below)
+            if (!h16 && !pl.gx_in_place && !cl_in)
                 TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
                              launch_from_channels_last(dt, gx_cl, grad_input, nullptr, g.B, g.C, g.Sn, s));
-            else if (!pl.gx_in_place)
+            else if (!h16 && !pl.gx_in_place)
                 TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
                              launch_acc_to_storage(dt, gx_cl, grad_input, (size_t)g.B * g.Sn * g.C, s));
         } else {
             void *wf = at(workspace, L.wf);
             if (pl.fw.ok) {
                 void *w16 = sampled16 ? at(workspace, L.w16) : nullptr;
-                if (w16 != nullptr)
+                if (!h16 && w16 != nullptr)
                     TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fwd_win_layout16(dt, g, pl.fw, weight, w16, flag, s, wf));
-                else
+                else if (!h16)
                     TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_fwd_win_layout(dt, g, pl.fw, weight, wf, s));
                 TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,
                              launch_fwd_win(dt, pl.dim, g, pl.wn_f, pl.fw, xcl, wf, w16, flag, offset, mask, nullptr,
@@ -794,7 +862,22 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
     if (gmask && (desc->flags & TVDCN_FLAG_MASK_SOFTMAX))
         TVDCN_LAUNCH(TVDCN_KERNEL_MASK_SOFTMAX, s,
                      launch_mask_softmax_logit_grad(dt, mask, gmask, (int64_t)g.B * g.mg, g.Kn, g.Pn, s));
-    if (!direct && !pl.few.ok && (goff || gmask))
+    if (!direct && pl.wn_s.ok) {
+        Out16 o{};
+        o.acc = pl.transposed ? nullptr : at(workspace, L.cl_acc);
+        o.y = grad_input;
+        o.cl = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
+        o.B = g.B;
+        o.C = g.C;
+        o.S = g.Sn;
+        o.a0 = goff;
+        o.o0 = grad_offset;
+        o.n0 = n_goff;
+        o.a1 = gmask;
+        o.o1 = grad_mask;
+        o.n1 = n_gmask;
+        TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_out16(dt, o, s));
+    } else if (!direct && !pl.few.ok && (goff || gmask))
         TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s,
                      launch_acc_to_storage2(dt, goff, grad_offset, goff ? n_goff : 0, gmask, grad_mask,
                                             gmask ? n_gmask : 0, s));

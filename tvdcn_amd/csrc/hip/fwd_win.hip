@@ -21,7 +21,7 @@
 // of the next slice (prefetched into registers during the last step of the current
 // one) replaces the current one, and where the sampling table is rebuilt (when the
 // offset / mask group changes). See window.h for the tile / window machinery.
-#include "window.h"
+#include "operands.h"
 
 namespace tvdcn_hip {
 namespace {
@@ -107,7 +107,8 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     const bool deformable = offset != nullptr;
     const int slices = (g.Cg + BC - 1) / BC;
     // the 16-bit loop when its weight was laid out and (fp32) no operand was flagged
-    const bool use16_flag = w16 != nullptr && (flag == nullptr || *flag == 0);
+    // (fp16 / bf16: always)
+    const bool use16_flag = npiece_of<T>() == 1 || (w16 != nullptr && (flag == nullptr || *flag == 0));
     // fp32 as fp16 pieces: the sampled columns' scale, and the one back out (the weight's with it)
     const int s_b = npiece_of<T>() == 2 && use16_flag ? sampled_scale(g, flag, mask != nullptr) : 0;
     const int s_back = npiece_of<T>() == 2 && use16_flag ? -(s_b + operand_scale(flag, AMAX_W)) : 0;
@@ -700,46 +701,13 @@ __global__ void fwd_win_weight_kernel(const T *__restrict__ w, float *__restrict
     fwd_weight_f32<T>(w, wp, G, Mg, Cg, Kn, slices, Mg_pad);
 }
 
-// weight (M, Cg, Kn) -> W16[G][slices][pp][Mg_pad / 16][NP][64 lanes][8]: per (slice, tap pair j
-// of pass p, 16-row block) the 16x16x32 A fragments: lane l = m % 16 + 16 q holds at e = 0..7
-// W[m][slice * 16 + 4 q + e % 4] at tap p * tpp + 2 j + e / 4 (zero past the pass, Mg, Cg); fp32
-// as two fp16 pieces at the weight's scale (*flag set for a value bad for the split), fp16 / bf16
-// as they are
-// (wp: when not null, the fp32 layout of fwd_win_weight_kernel is written by the same launch)
+// the weight as W16 (w16_block) and, wp, in the fp32 loop's layout, in one launch
 template <typename T, int NP>
 __global__ void __launch_bounds__(256)
 fwd_w16_kernel(const T *__restrict__ w, uint16_t *__restrict__ out, int *flag, int G, int Mg, int Cg, int Kn, int slices,
                int nmb, int tpp, int hp, int pp, float *__restrict__ wp) {
     if (wp != nullptr) fwd_weight_f32<T>(w, wp, G, Mg, Cg, Kn, slices, nmb * 16);
-    const unsigned total = (unsigned)G * slices * pp * nmb * 64;
-    const int sw = NP == 2 ? operand_scale(flag, AMAX_W) : 0;
-    bool bad = false;
-    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        const int l = (int)(i & 63);
-        unsigned r = i >> 6;
-        const int mb = (int)(r % nmb);
-        r /= nmb;
-        const int pq = (int)(r % pp);
-        r /= pp;
-        const int cs = (int)(r % slices);
-        const int grp = (int)(r / slices);
-        const int pass = pq / hp, j = pq - pass * hp;
-        const int tf = pass * tpp, ntp = min(tpp, Kn - tf);
-        const int m = mb * 16 + (l & 15), q = l >> 4;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int tl = 2 * j + (e >> 2), c = cs * BC + 4 * q + (e & 3);
-            v[e] = (tl < ntp && m < Mg && c < Cg) ? to_acc<float>(w[(((size_t)grp * Mg + m) * Cg + c) * Kn + tf + tl]) : 0.f;
-            bad = bad || split_bad(v[e]);
-        }
-        uint4 o[NP];
-        pack8_16<T, NP>(v, sw, o);
-        uint16_t *dst = out + ((((size_t)grp * slices + cs) * pp + pq) * nmb + mb) * (NP * 512) + l * 8;
-#pragma unroll
-        for (int k = 0; k < NP; ++k) *reinterpret_cast<uint4 *>(dst + k * 512) = o[k];
-    }
-    if (NP == 2 && bad) atomicOr(flag, 1);
+    w16_block<T, NP>(blockIdx.x, gridDim.x, w, out, flag, G, Mg, Cg, Kn, slices, nmb, tpp, hp, pp);
 }
 
 template <int DIM, typename T, int MB, bool STAGE>
@@ -897,9 +865,7 @@ hipError_t launch_fwd_win_layout(int dtype, const Geo &g, const FwdWin &fw, cons
                        static_cast<float *>(wp), g.G, g.Mg, g.Cg, g.Kn, slices, fw.Mg_pad);                      \
     return hipGetLastError();
     switch (dtype) {
-        case kF32: { TVDCN_FWL(float) }
-        case kF16: { TVDCN_FWL(__half) }
-        case kBF16: { TVDCN_FWL(__hip_bfloat16) }
+        case kF32: { TVDCN_FWL(float) }   // (fp16 / bf16 run no fp32 loop)
     }
 #undef TVDCN_FWL
     return hipErrorInvalidValue;
@@ -920,9 +886,7 @@ hipError_t launch_fwd_win_layout16(int dtype, const Geo &g, const FwdWin &fw, co
                        fw.hp, fw.pp, static_cast<float *>(wp));                                                        \
     return hipGetLastError();
     switch (dtype) {
-        case kF32: { TVDCN_FW16(float, npiece_of<float>()) }
-        case kF16: { TVDCN_FW16(__half, npiece_of<__half>()) }
-        case kBF16: { TVDCN_FW16(__hip_bfloat16, npiece_of<__hip_bfloat16>()) }
+        case kF32: { TVDCN_FW16(float, npiece_of<float>()) }   // (fp16 / bf16: launch_prep16)
     }
 #undef TVDCN_FW16
     return hipErrorInvalidValue;
@@ -953,6 +917,7 @@ hipError_t launch_fwd_win(int dtype, int dim, const Geo &g, const WinTiles &wt, 
                           const void *wf, const void *w16, const int *flag, const void *offset, const void *mask,
                           const void *bias, void *y, void *y32, hipStream_t s) {
     if (fw_.ksplit != 1 && y32 == nullptr) return hipErrorInvalidValue;
+    if (dtype != kF32 && w16 == nullptr) return hipErrorInvalidValue;
     if (g.B == 0) return hipSuccess;
     // (a batch block's output may be less aligned than the caller's)
     const size_t quad = 4 * (dtype == kF32 ? sizeof(float) : sizeof(uint16_t));

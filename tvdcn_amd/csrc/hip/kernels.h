@@ -233,6 +233,37 @@ hipError_t launch_bwd_data(int dtype, int dim, const Geo &g, const DataTiles &t,
 // 16-bit loop (needs WeightWin::z8)
 hipError_t launch_data_win_prep(int dtype, const Geo &g, const WinTiles &t, const void *z, const void *w, void *zs,
                                 void *wsplit, void *wd, int *flag, hipStream_t s, void *zw = nullptr);
+// fp16 / bf16: the layouts of a call in one launch (prep16.hip); jobs with null pointers are left out
+struct Prep16 {
+    const void *x;       // sampled tensor -> xcl, float channels-last (x_cl: x is channels-last already)
+    bool x_cl;
+    void *xcl;
+    const void *z, *w;   // z: with w, the data gradient's operands zs, wsplit and (may be null) zw, as
+    void *zs, *wsplit, *zw;   // launch_data_win_prep, over the tiling wt
+    const WinTiles *wt;
+    void *w16;           // w as the windowed forward's operands, over fw
+    const FwdWin *fw;
+    const void *gout;    // gb = (accumulate: gb +) the bias gradient of gout's bias_c channels of bias_s positions
+    void *gb;
+    int bias_c, bias_s;
+    bool accumulate;
+    void *fill[3];       // float accumulators to zero (16-byte aligned, room to a multiple of four)
+    size_t fill_n[3];
+};
+hipError_t launch_prep16(int dtype, const Geo &g, const Prep16 &j, hipStream_t s);
+// fp16 / bf16: float accumulators into the caller's tensors, one launch: acc (B, *S, C) into y, NC<spatial> (+
+// bias, may be null) or, cl, in its own order; a0 / a1 elementwise into o0 / o1. Null sources are left out.
+struct Out16 {
+    const void *acc;
+    void *y;
+    const void *bias;
+    bool cl;
+    int B, C, S;
+    const void *a0, *a1;
+    void *o0, *o1;
+    size_t n0, n1;
+};
+hipError_t launch_out16(int dtype, const Out16 &j, hipStream_t s);
 // gx_nchw: gx_cl is grad_input as the caller's float32 (B, C, *S) tensor (zeroed), not the
 // channels-last accumulator
 hipError_t launch_bwd_data_win(int dtype, int dim, const Geo &g, const WinTiles &t, bool scatter, bool coord,
