@@ -195,9 +195,9 @@ bwd_weight_win_kernel(const Geo g, const WinTiles wt, const WeightWin ww, const 
                         const acc4 r = geo[tl * BPX + i];
                         acc4 sv[4];
                         if (nq == 4)
-                            sample3_all_fix<true>(g, wt, tile, xwin, xb, 4, r, deformable, sv);
+                            sample3_all<true>(g, wt, tile, xwin, xb, 4, r, deformable, sv);
                         else
-                            sample3_all_fix<false>(g, wt, tile, xwin, xb, nq, r, deformable, sv);
+                            sample3_all<false>(g, wt, tile, xwin, xb, nq, r, deformable, sv);
                         float *row = dst + tl * BC * SS + sj;
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
@@ -290,9 +290,9 @@ bwd_weight_win_kernel(const Geo g, const WinTiles wt, const WeightWin ww, const 
                             const acc4 r = geo[tl * BPX + i];
                             acc4 sv[4];
                             if (nq == 4)
-                                sample3_all_fix<true>(g, wt, tile, xwin, xb, 4, r, deformable, sv);
+                                sample3_all<true>(g, wt, tile, xwin, xb, 4, r, deformable, sv);
                             else
-                                sample3_all_fix<false>(g, wt, tile, xwin, xb, nq, r, deformable, sv);
+                                sample3_all<false>(g, wt, tile, xwin, xb, nq, r, deformable, sv);
 #pragma unroll
                             for (int j = 0; j < 4; ++j)
 #pragma unroll

@@ -77,8 +77,14 @@ __device__ __forceinline__ void store_frag(const Geo &g, T *yg, int m0, int p, b
     }
 }
 
-// STAGE: the 16-bit loop's weight blocks are staged in LDS (1D / 2D, fw.stage_bytes > 0)
-template <int DIM, typename T, int MB, bool STAGE>
+// STAGE: the 16-bit loop's weight blocks are staged in LDS (1D / 2D, fw.stage_bytes > 0). USE16: the 16x16x32
+// MFMA loop; an fp32 call launches both instantiations and the operand flag has one return at once. ONE: a
+// single pass of taps. Either loop beside the other, or beside a loop over the passes, cost the 2D kernel 75
+// registers and 226 spilled scalars (174 and none without), the compiler keeping both loops' and all phases'
+// values live. (always_inline: at this size
+// the inliner otherwise leaves the lambdas as calls.) us a call: 256 channels, k3, 8 x 64x64, float32 training
+// 843 -> 839, bfloat16 128 channels, 2 x 100x152 inference 107 -> 103.
+template <int DIM, typename T, int MB, bool STAGE, bool USE16, bool ONE>
 __global__ void __launch_bounds__(NT)
 fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__restrict__ xcl,
                const float *__restrict__ wf, const uint16_t *__restrict__ w16, const int *flag,
@@ -106,12 +112,10 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     const int grp = L / n_sp;
     const bool deformable = offset != nullptr;
     const int slices = (g.Cg + BC - 1) / BC;
-    // the 16-bit loop when its weight was laid out and (fp32) no operand was flagged
-    // (fp16 / bf16: always)
-    const bool use16_flag = npiece_of<T>() == 1 || (w16 != nullptr && (flag == nullptr || *flag == 0));
+    if (npiece_of<T>() == 2 && flag != nullptr && (*flag == 0) != USE16) return;   // the other launch's
     // fp32 as fp16 pieces: the sampled columns' scale, and the one back out (the weight's with it)
-    const int s_b = npiece_of<T>() == 2 && use16_flag ? sampled_scale(g, flag, mask != nullptr) : 0;
-    const int s_back = npiece_of<T>() == 2 && use16_flag ? -(s_b + operand_scale(flag, AMAX_W)) : 0;
+    const int s_b = npiece_of<T>() == 2 && USE16 ? sampled_scale(g, flag, mask != nullptr) : 0;
+    const int s_back = npiece_of<T>() == 2 && USE16 ? -(s_b + operand_scale(flag, AMAX_W)) : 0;
     // the sampling table's masks carry 2^s_b, so that the B fragments come out of the sampling at
     // their pieces' scale
     const float mscale_b = ldexpf(1.f, s_b);
@@ -119,10 +123,18 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // [cs_lo, cs_hi) of them
     const int u_lo = ks * fw.units_per;
     int cs_lo = 0, cs_hi = 0;
-    auto pass_slices = [&](int pass) {
+    auto pass_slices = [&](int pass) __attribute__((always_inline)) {
         cs_lo = max(u_lo - pass * slices, 0);
         cs_hi = min(u_lo + fw.units_per - pass * slices, slices);
         return cs_lo < cs_hi;
+    };
+    auto passes = [&](auto &&body) __attribute__((always_inline)) {
+        if constexpr (ONE) {
+            if (pass_slices(0)) body(0, g.Kn);
+        } else {
+            for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass)
+                if (pass_slices(pass)) body(t0, min(wt.tpp, g.Kn - t0));
+        }
     };
 
     Tile tile;
@@ -137,7 +149,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // cells (and their grid indices) are the same for every slice: resolved once.
     // (3D resolves them at each fill: its registers are taken by the B fragments of a tap group)
     int xsi[XQ];   // flat sampled-grid index of the thread's cells (-1: outside the grid / window)
-    auto resolve_cells = [&]() {
+    auto resolve_cells = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < XQ; ++j) {
             const int e = tid + j * NT;
@@ -146,7 +158,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     };
     if constexpr (DIM != 3) resolve_cells();
     acc4 xpre[XQ];
-    auto prefetch_x = [&](int cs) {
+    auto prefetch_x = [&](int cs) __attribute__((always_inline)) {
         const float *xb = xg + cs * BC + 4 * (tid & 3);
         const bool q_ok = cs * BC + 4 * (tid & 3) < g.Cg;   // quad of thread tid + j * NT is tid % 4
 #pragma unroll
@@ -155,7 +167,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
             if (xsi[j] >= 0 && q_ok) xpre[j] = *reinterpret_cast<const acc4 *>(xb + (size_t)xsi[j] * g.C);
         }
     };
-    auto store_x = [&]() {
+    auto store_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < XQ; ++j) {
             const int e = tid + j * NT;
@@ -165,7 +177,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
 
     // B fragment of pixel block pb for (slice cs, tap tl of the pass): the sampled values of
     // channels cs * 16 + 4 * (lane / 16) .. + 3 at pixel wave * 32 + pb * 16 + lane % 16
-    auto build_b = [&](int cs, int tl, acc4 (&bv)[PB]) {
+    auto build_b = [&](int cs, int tl, acc4 (&bv)[PB]) __attribute__((always_inline)) {
         const int qd = q;
         const bool q_ok = cs * BC + 4 * qd < g.Cg;
 #pragma unroll
@@ -215,8 +227,8 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // is one contiguous 1 KB wave load; consecutive taps of a slice are adjacent.
     const size_t step_elems = (size_t)fw.Mg_pad * BC;
     const float *wlane = wf + (size_t)grp * slices * g.Kn * step_elems + (size_t)mt * MB * 256 + (lane & 15) * BC + 4 * q;
-    auto wptr = [&](int cs, int t) { return wlane + ((size_t)cs * g.Kn + t) * step_elems; };
-    auto load_w = [&](const float *p, acc4 (&wr)[MB]) {
+    auto wptr = [&](int cs, int t) __attribute__((always_inline)) { return wlane + ((size_t)cs * g.Kn + t) * step_elems; };
+    auto load_w = [&](const float *p, acc4 (&wr)[MB]) __attribute__((always_inline)) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) wr[mb] = *reinterpret_cast<const acc4 *>(p + mb * 256);
     };
@@ -230,7 +242,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // MFMAs of one step with B fragments bv and A fragments wr; each row block's fragment
     // is reloaded from pn (the next step's, or this step's own at the end of a pass) right
     // after its last use (issue order pinned)
-    auto mfma_step = [&](const acc4 (&bv)[PB], acc4 (&wr)[MB], const float *pn) {
+    auto mfma_step = [&](const acc4 (&bv)[PB], acc4 (&wr)[MB], const float *pn) __attribute__((always_inline)) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
@@ -245,7 +257,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     // switch the tables to slice cs: X window from the prefetch registers, sampling
     // table rebuilt when the slice's offset / mask group differs from the last one
     int geo_og = -1, geo_mg = -1;
-    auto open_slice = [&](int cs, int t0, int ntaps) {
+    auto open_slice = [&](int cs, int t0, int ntaps) __attribute__((always_inline)) {
         if constexpr (DIM == 3) {
             resolve_cells();
             prefetch_x(cs);
@@ -269,7 +281,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     //      pass), split into pieces for fp32 and rounded to T otherwise (the reference's columns
     //      of a half-precision input are half). W16 holds the A fragments in the same K order.
     //      The weight blocks are staged in LDS (below).
-    auto pass16 = [&](int t0, int ntaps) {
+    auto pass16 = [&](int t0, int ntaps) __attribute__((always_inline)) {
         if constexpr (DIM < 3) {
             constexpr int NP = npiece_of<T>();
             const int npair = (ntaps + 1) >> 1;
@@ -279,10 +291,10 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
             const int pp0 = (t0 / wt.tpp) * fw.hp;
             // (the step's block: wave-uniform; lanes add their offsets when they load)
             const uint16_t *wl = w16 + (size_t)mt * MB * (NP * 512);
-            auto wptr16 = [&](int cs, int j) {
+            auto wptr16 = [&](int cs, int j) __attribute__((always_inline)) {
                 return wl + (((size_t)grp * slices + cs) * fw.pp + pp0 + j) * nmb * (NP * 512);
             };
-            auto build_pair = [&](int cs, int j, uint4 (&bp)[PB][NP]) {
+            auto build_pair = [&](int cs, int j, uint4 (&bp)[PB][NP]) __attribute__((always_inline)) {
                 acc4 b0[PB], b1[PB];
                 build_b(cs, 2 * j, b0);
                 if (2 * j + 1 < ntaps) {
@@ -312,7 +324,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 uint16_t *wst = reinterpret_cast<uint16_t *>(xwin + (size_t)wt.cells * XS);   // [2][U][WBLK]
                 // (slice, pair) of the next step to stage, advanced step by step (no divisions)
                 int s_cs = cs_lo, s_j = 0;
-                auto stage_unit = [&](int u, int buf) {
+                auto stage_unit = [&](int u, int buf) __attribute__((always_inline)) {
 #pragma unroll
                     for (int su = 0; su < U; ++su) {
                         const int k = u * U + su;
@@ -327,14 +339,14 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                             __builtin_amdgcn_global_load_lds(blk + i * 512 + lane * 8, dst + i * 512, 16, 0, 0);
                     }
                 };
-                auto load_w16 = [&](const uint16_t *blk, int mb, uint4 (&f)[NP]) {
+                auto load_w16 = [&](const uint16_t *blk, int mb, uint4 (&f)[NP]) __attribute__((always_inline)) {
                     const uint16_t *p = blk + mb * (NP * 512) + lane * 8;
 #pragma unroll
                     for (int k = 0; k < NP; ++k) f[k] = *reinterpret_cast<const uint4 *>(p + k * 512);
                 };
                 // MFMAs of one step on its staged block; block mb + 1's fragments are read before
                 // block mb's MFMAs
-                auto mfma_pair = [&](const uint4 (&bv)[PB][NP], uint4 (&wa)[2][NP], const uint16_t *blk) {
+                auto mfma_pair = [&](const uint4 (&bv)[PB][NP], uint4 (&wa)[2][NP], const uint16_t *blk) __attribute__((always_inline)) {
                     load_w16(blk, 0, wa[0]);
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
@@ -346,7 +358,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                     }
                 };
                 // the staged unit's loads done, then the workgroup barrier that publishes it
-                auto publish = [&]() {
+                auto publish = [&]() __attribute__((always_inline)) {
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __syncthreads();
                 };
@@ -385,14 +397,14 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
             } else {
                 // (the weight's staging would cost the window its margin: fragments straight from
                 // global memory, each row block's loaded one block ahead)
-                auto load_w16g = [&](const uint16_t *p, uint4 (&f)[NP]) {
+                auto load_w16g = [&](const uint16_t *p, uint4 (&f)[NP]) __attribute__((always_inline)) {
 #pragma unroll
                     for (int k = 0; k < NP; ++k) f[k] = *reinterpret_cast<const uint4 *>(p + lane * 8 + k * 512);
                 };
                 // MFMAs of one step; block mb + 1's fragments (the next step's block 0 at the end)
                 // are loaded before block mb's MFMAs
                 auto mfma_pair_g = [&](const uint4 (&bv)[PB][NP], uint4 (&wa)[2][NP], const uint16_t *pcur,
-                                       const uint16_t *pnext) {
+                                       const uint16_t *pnext) __attribute__((always_inline)) {
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
                         load_w16g(mb + 1 < MB ? pcur + (size_t)(mb + 1) * (NP * 512) : pnext, wa[(mb + 1) & 1]);
@@ -436,7 +448,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
         // all 16 channels of the slice (the corner geometry formed once per (pixel, tap)
         // rather than once per channel quad); a row transpose then gives every lane its
         // channel quad of the group's four taps, the B fragments of four steps.
-        auto build_group = [&](int cs, int tg, int ntaps, acc4 (&bq)[4][PB]) {
+        auto build_group = [&](int cs, int tg, int ntaps, acc4 (&bq)[4][PB]) __attribute__((always_inline)) {
             const int tl = tg * 4 + q;
             const int nq = min(4, (g.Cg - cs * BC) >> 2);   // channel quads of the slice in the group
 #pragma unroll
@@ -456,7 +468,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 for (int j = 0; j < 4; ++j) bq[j][pb] = sv[j];
             }
         };
-        if (use16_flag) {
+        if constexpr (USE16) {
             // 16x16x32 steps: a group's four taps are two tap pairs, each pair's B fragment its
             // two sampled quads (the 16-bit loop's K order, W16 below), split into pieces (fp32)
             // or rounded to T; the pair's A fragments come from global memory, each row block's
@@ -464,19 +476,17 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
             constexpr int NP = npiece_of<T>();
             const int nmb = fw.Mg_pad / 16;
             const uint16_t *wl = w16 + (size_t)mt * MB * (NP * 512);
-            auto load_w16g = [&](const uint16_t *p, uint4 (&f)[NP]) {
+            auto load_w16g = [&](const uint16_t *p, uint4 (&f)[NP]) __attribute__((always_inline)) {
 #pragma unroll
                 for (int k = 0; k < NP; ++k) f[k] = *reinterpret_cast<const uint4 *>(p + lane * 8 + k * 512);
             };
             static_assert(MB % 2 == 0, "row blocks in pairs: the next step's block 0 lands in slot 0");
-            for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
-                if (!pass_slices(pass)) continue;
-                const int ntaps = min(wt.tpp, g.Kn - t0);
+            passes([&](int t0, int ntaps) __attribute__((always_inline)) {
                 const int ngr = (ntaps + 3) >> 2;
                 const int ngroups = (cs_hi - cs_lo) * ngr;
                 geo_og = geo_mg = -1;
                 const int pp0 = (t0 / wt.tpp) * fw.hp;
-                auto wptr16 = [&](int cs, int j) {
+                auto wptr16 = [&](int cs, int j) __attribute__((always_inline)) {
                     return wl + (((size_t)grp * slices + cs) * fw.pp + pp0 + j) * nmb * (NP * 512);
                 };
                 uint4 wa[2][NP];
@@ -524,11 +534,9 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                     cs = csn;
                     tg = tgn;
                 }
-            }
+            });
         } else {
-            for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
-                if (!pass_slices(pass)) continue;
-                const int ntaps = min(wt.tpp, g.Kn - t0);
+            passes([&](int t0, int ntaps) __attribute__((always_inline)) {
                 const int ngr = (ntaps + 3) >> 2;   // tap groups per slice
                 const int ngroups = (cs_hi - cs_lo) * ngr;
                 geo_og = geo_mg = -1;   // a new pass of taps: the table must be rebuilt
@@ -569,15 +577,12 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                     cs = csn;
                     tg = tgn;
                 }
-            }
+            });
         }
-    } else if (use16_flag) {
-        for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass)
-            if (pass_slices(pass)) pass16(t0, min(wt.tpp, g.Kn - t0));
+    } else if constexpr (USE16) {
+        passes(pass16);
     } else {
-        for (int t0 = 0, pass = 0; t0 < g.Kn; t0 += wt.tpp, ++pass) {
-            if (!pass_slices(pass)) continue;
-            const int ntaps = min(wt.tpp, g.Kn - t0);
+        passes([&](int t0, int ntaps) __attribute__((always_inline)) {
             const int nsteps = (cs_hi - cs_lo) * ntaps;
             geo_og = geo_mg = -1;   // a new pass of taps: the table must be rebuilt
 
@@ -613,7 +618,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 cs = csn;
                 tl = tln;
             }
-        }
+        });
     }
 
     // ---- epilogue: + bias, store NC<spatial>. With several shares each stores its fp32 partial to
@@ -710,11 +715,11 @@ fwd_w16_kernel(const T *__restrict__ w, uint16_t *__restrict__ out, int *flag, i
     w16_block<T, NP>(blockIdx.x, gridDim.x, w, out, flag, G, Mg, Cg, Kn, slices, nmb, tpp, hp, pp);
 }
 
-template <int DIM, typename T, int MB, bool STAGE>
-hipError_t launch_k(const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl, const void *wf,
+template <int DIM, typename T, int MB, bool STAGE, bool USE16, bool ONE>
+hipError_t launch_k1(const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl, const void *wf,
                     const void *w16, const int *flag, const void *offset, const void *mask, const void *bias, void *y,
                     void *y32, hipStream_t s) {
-    auto kern = fwd_win_kernel<DIM, T, MB, STAGE>;
+    auto kern = fwd_win_kernel<DIM, T, MB, STAGE, USE16, ONE>;
     const size_t lds = ((size_t)GEO_WORDS + (size_t)(wt.cells + (DIM == 3)) * XS) * sizeof(float) + fw.stage_bytes;
     static std::atomic<unsigned long long> lds_raised{0};   // per device, see raise_lds_limit
     if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
@@ -725,6 +730,24 @@ hipError_t launch_k(const Geo &g, const WinTiles &wt, const FwdWin &fw, const vo
                        static_cast<const T *>(offset), static_cast<const T *>(mask),
                        static_cast<const T *>(bias), static_cast<T *>(y), static_cast<float *>(y32));
     return hipGetLastError();
+}
+
+// the 16-bit loop (when its weight was laid out) and, fp32, the fp32 loop beside it (4.5 us when not selected)
+template <int DIM, typename T, int MB, bool STAGE>
+hipError_t launch_k(const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl, const void *wf,
+                    const void *w16, const int *flag, const void *offset, const void *mask, const void *bias, void *y,
+                    void *y32, hipStream_t s) {
+    if (w16 != nullptr) {
+        const hipError_t e =
+            g.Kn <= wt.tpp
+                ? launch_k1<DIM, T, MB, STAGE, true, true>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s)
+                : launch_k1<DIM, T, MB, STAGE, true, false>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+        if (e != hipSuccess || npiece_of<T>() == 1 || flag == nullptr) return e;
+    }
+    if constexpr (npiece_of<T>() == 2)
+        return launch_k1<DIM, T, MB, STAGE, false, false>(g, wt, fw, xcl, wf, w16, w16 != nullptr ? flag : nullptr, offset,
+                                                          mask, bias, y, y32, s);
+    return hipErrorInvalidValue;
 }
 
 template <int DIM, typename T>

@@ -149,137 +149,11 @@ __device__ __forceinline__ acc4 window_sample_masked(const WinTiles &wt, const f
 }
 
 // Corner geometry of a 3D record (absolute positions) against the tile's window and the
-// sampled grid: per axis the low corner, the high-corner weight and whether each of the two
-// corner coordinates lies in the window / in the grid. Corner k = (z bit, y bit, x bit) sits at
-// window cell cell0 + bz * WE_y * WE_x + by * WE_x + bx and grid index idx0 + bz * S_y * S_x +
-// by * S_x + bx. Offset-free sampling (integer positions) has only the low corner.
-struct Corners3 {
-    float fh[3];
-    bool win[3][2], grid[3][2];
-    int cell0, idx0;
-    bool inside;   // sample range rule: -1 < pos < S on every axis
-    __device__ __forceinline__ Corners3(const Geo &g, const WinTiles &wt, const Tile &tile, const acc4 &r,
-                                        bool deformable) {
-        int lo[3], wl[3];
-        inside = true;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float f = floorf(r[a]);
-            lo[a] = (int)f;
-            fh[a] = deformable ? r[a] - f : 0.f;
-            inside = inside && r[a] > -1.f && r[a] < (float)g.S[a];
-            wl[a] = lo[a] - tile.org[a];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                win[a][b] = (unsigned)(wl[a] + b) < (unsigned)wt.WE[a];
-                grid[a][b] = (unsigned)(lo[a] + b) < (unsigned)g.S[a];
-            }
-        }
-        cell0 = (wl[0] * wt.WE[1] + wl[1]) * wt.WE[2] + wl[2];
-        idx0 = (lo[0] * g.S[1] + lo[1]) * g.S[2] + lo[2];
-    }
-    __device__ __forceinline__ bool in_win(int k) const { return win[0][k >> 2] && win[1][(k >> 1) & 1] && win[2][k & 1]; }
-    __device__ __forceinline__ bool in_grid(int k) const {
-        return grid[0][k >> 2] && grid[1][(k >> 1) & 1] && grid[2][k & 1];
-    }
-    __device__ __forceinline__ int cell(const WinTiles &wt, int k) const {
-        return cell0 + (k >> 2) * (wt.WE[1] * wt.WE[2]) + ((k >> 1) & 1) * wt.WE[2] + (k & 1);
-    }
-    __device__ __forceinline__ int idx(const Geo &g, int k) const {
-        return idx0 + (k >> 2) * (g.S[1] * g.S[2]) + ((k >> 1) & 1) * g.S[2] + (k & 1);
-    }
-    // trilinear weight of corner k (product in the reference's axis order)
-    __device__ __forceinline__ float weight(int k) const {
-        const float wz = (k >> 2) ? fh[0] : 1.f - fh[0];
-        const float wy = ((k >> 1) & 1) ? fh[1] : 1.f - fh[1];
-        const float wx = (k & 1) ? fh[2] : 1.f - fh[2];
-        return wz * wy * wx;
-    }
-};
-
-// X of one channel quad at corner k: from the window when the corner lies in it (window
-// cells outside the grid hold zeros), else from global memory (xgq: the channels-last X of
-// the tile's image at the quad's first channel), zero outside the grid. The LDS read is
-// unconditional (clamped) and the global read sits in its own branch: the two address
-// spaces are never merged into one pointer.
-__device__ __forceinline__ acc4 corner_x3(const Geo &g, const WinTiles &wt, const Corners3 &cr, int k, const float *xwin,
-                                          int xq, const float *__restrict__ xgq, bool q_ok, bool xglobal = false) {
-    const bool iw = !xglobal && cr.in_win(k);
-    acc4 x = *reinterpret_cast<const acc4 *>(xwin + (iw ? cr.cell(wt, k) : 0) * XS + xq);
-    if (!iw) {
-        x = acc4{0.f, 0.f, 0.f, 0.f};
-        if (q_ok && cr.in_grid(k)) x = *reinterpret_cast<const acc4 *>(xgq + (size_t)cr.idx(g, k) * g.C);
-    }
-    return x;
-}
-
-// mask * sample of one channel quad at a 3D record: one branch-light path for every lane
-// (the 3D windows that fit in LDS have margins of about one cell, so most waves hold some
-// lane with a corner outside the window; a separate in-window fast path would run beside
-// this one rather than instead of it).
-__device__ __forceinline__ acc4 sample3_masked(const Geo &g, const WinTiles &wt, const Tile &tile, const float *xwin,
-                                               int xq, const float *__restrict__ xgq, bool q_ok, const acc4 &r,
-                                               bool deformable) {
-    const Corners3 cr(g, wt, tile, r, deformable);
-    acc4 sv = acc4{0.f, 0.f, 0.f, 0.f};
-    if (!cr.inside) return sv;
-    const float mk = r[3];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (k > 0 && !deformable) break;
-        sv += (mk * cr.weight(k)) * corner_x3(g, wt, cr, k, xwin, xq, xgq, q_ok);
-    }
-    return sv;
-}
-
-// mask * sample of all 16 channels of the tile's slice at a 3D record: s[j] = channels
-// 4j .. 4j + 3 (xgs: the channels-last X of the tile's image at the slice's first channel;
-// nq: channel quads of the slice inside the group, 4 when FULLQ). The corner geometry and
-// the eight mask-folded weights are formed once for the 16 channels. Window cell wt.cells
-// must hold zeros (the zero cell): a corner outside the window reads it, and a corner
-// outside the window but inside the grid then overwrites it with the global values.
-template <bool FULLQ>
-__device__ __forceinline__ void sample3_all(const Geo &g, const WinTiles &wt, const Tile &tile, const float *xwin,
-                                            const float *__restrict__ xgs, int nq, const acc4 &r, bool deformable,
-                                            acc4 (&s)[4]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s[j] = acc4{0.f, 0.f, 0.f, 0.f};
-    const Corners3 cr(g, wt, tile, r, deformable);
-    if (!cr.inside) return;
-    auto corner = [&](int k, float w) {
-        const bool iw = cr.in_win(k);
-        const float *xc = xwin + (iw ? cr.cell(wt, k) : wt.cells) * XS;
-        acc4 x[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const acc4 *>(xc + 4 * j);
-        if (!iw && cr.in_grid(k)) {
-            const float *xp = xgs + (size_t)cr.idx(g, k) * g.C;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (FULLQ || j < nq) x[j] = *reinterpret_cast<const acc4 *>(xp + 4 * j);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[j] += w * x[j];
-    };
-    const float mk = r[3];
-    if (deformable) {
-        // mask-folded trilinear weights: (z, y) pairs first, then x
-        const float z1 = mk * cr.fh[0], z0 = mk - z1;
-        const float zy[4] = {z0 - z0 * cr.fh[1], z0 * cr.fh[1], z1 - z1 * cr.fh[1], z1 * cr.fh[1]};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float w1 = zy[j] * cr.fh[2];
-            corner(2 * j, zy[j] - w1);
-            corner(2 * j + 1, w1);
-        }
-    } else {
-        corner(0, mk);   // offset-free sampling: the low corner only
-    }
-}
-
-// The corner geometry of Corners3 with the window / grid membership of the eight corners as
-// 8-bit lane masks (bit k: corner k) held in a vector register, for the branch-free sampler
-// below.
+// sampled grid: the low corner and the high-corner weight per axis, and the window / grid
+// membership of the eight corners as 8-bit lane masks (bit k: corner k = (z bit, y bit, x
+// bit)) in a vector register. Corner k sits at window cell cell0 + bz * WE_y * WE_x + by * WE_x
+// + bx and grid index idx0 + bz * S_y * S_x + by * S_x + bx. Offset-free sampling (integer
+// positions) has only the low corner.
 struct Corners3M {
     float fh[3];
     int cell0, idx0;
@@ -317,13 +191,17 @@ struct Corners3M {
 
 };
 
-// sample3_all with every corner read from the window without a branch -- a corner outside it
-// reads window cell wt.cells, which must hold zeros (the zero cell) -- and the corners inside the
-// grid but outside the window added from global memory afterwards (a sample outside the range
-// rule reads zero cells only, whatever its mask). Fewer registers than sample3_all; measured
-// faster for the weight gradient's S tiles, slower for the forward's B fragments.
+// mask * sample of all 16 channels of the tile's slice at a 3D record: s[j] = channels
+// 4j .. 4j + 3 (xgs: the channels-last X of the tile's image at the slice's first channel;
+// nq: channel quads of the slice inside the group, 4 when FULLQ). The corner geometry and
+// the eight mask-folded weights are formed once for the 16 channels. Every corner is read
+// from the window without a branch -- one outside it reads window cell wt.cells, which must
+// hold zeros (the zero cell) -- and the corners inside the grid but outside the window are added
+// from global memory afterwards (a sample outside the range rule reads zero cells only, whatever
+// its mask). A branch per corner, overwriting the window's values, held twelve lane conditions in
+// scalar pairs: ~500 spilled scalars and 52 spilled registers in the float32 forward.
 template <bool FULLQ>
-__device__ __forceinline__ void sample3_all_fix(const Geo &g, const WinTiles &wt, const Tile &tile, const float *xwin,
+__device__ __forceinline__ void sample3_all(const Geo &g, const WinTiles &wt, const Tile &tile, const float *xwin,
                                                 const float *__restrict__ xgs, int nq, const acc4 &r, bool deformable,
                                                 acc4 (&s)[4]) {
 #pragma unroll
