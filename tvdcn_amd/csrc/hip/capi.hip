@@ -759,6 +759,13 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         // the 16-bit loops of the sampled side (weight gradient; transposed: input gradient)
         const bool sampled16 = sampled16_host_ok(pl, desc) && (pl.ww.ok || (pl.transposed && pl.fw.ok));
         const void *x_in_place = nullptr;
+        // (fp32) the bias gradient rides on the layout copy too, where that has a block for every other
+        // channel (fewer would take the channels in turn)
+        const int bias_c = pl.transposed ? g.C : g.M, bias_s = pl.transposed ? g.Sn : g.Pn;
+        const BiasJob bj = {static_cast<const float *>(grad_out), static_cast<float *>(grad_bias), g.B, bias_c, bias_s,
+                            accumulate_weight, !pl.transposed};
+        const bool bias_in_copy = dt == kF32 && !cl_in && 2 * copy_blocks(g.C, g.Sn) >= bias_c &&
+                                  (grad_bias != nullptr || !pl.transposed);
         // (fp32) the 16-bit MFMA operands' largest magnitudes: the weight and X ride on X's layout
         // copy, Z = grad_out on the bias gradient (this block's, accumulated over the blocks),
         // whatever else on a launch of its own
@@ -767,7 +774,8 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
             const void *mchk = sampled16 ? mask_to_check(pl, desc, mask) : nullptr;
             TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, launch_to_channels_last(dt, X, xcl, g.B, g.C, g.Sn, s, flag, mchk,
                                                                          mask_numel(g), MASK_LIMIT, weight,
-                                                                         (size_t)g.M * g.Cg * g.Kn));
+                                                                         (size_t)g.M * g.Cg * g.Kn,
+                                                                         bias_in_copy ? &bj : nullptr));
         } else if (!h16) {
             if (direct)
                 x_in_place = xcl = const_cast<void *>(X);   // already the kernels' layout and type
@@ -777,10 +785,10 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         }
         // grad_out (B, Cout, *out_size): conv Cout = M on the column grid, transposed Cout = C on the
         // sampled grid
-        if (!h16 && !pl.transposed)
+        if (!h16 && !bias_in_copy && !pl.transposed)
             TVDCN_LAUNCH(TVDCN_KERNEL_BIAS_GRAD, s, launch_bias_grad(dt, grad_out, grad_bias, g.B, g.M, g.Pn, s,
                                                                      accumulate_weight, flag));
-        else if (!h16)
+        else if (!h16 && !bias_in_copy)
             TVDCN_LAUNCH(TVDCN_KERNEL_BIAS_GRAD, s, launch_bias_grad(dt, grad_out, grad_bias, g.B, g.C, g.Sn, s,
                                                                      accumulate_weight));
         TVDCN_LAUNCH(TVDCN_KERNEL_LAYOUT, s, operand_amax(pl, desc, cl_in ? weight : nullptr, cl_in ? X : nullptr,

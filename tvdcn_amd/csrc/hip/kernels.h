@@ -143,9 +143,20 @@ WeightTiles plan_weight(const Geo &g, int dtype);
 // launch, as launch_check_range does, its largest magnitude into the mask slot after *flag;
 // amax_w: fp32 only, when not null, the largest magnitudes of amax_w's amax_w_n values (the
 // weight slot) and of the copied values (the sampled-tensor slot), by the same launch)
+// (bias: fp32 only, the bias gradient of gout (B, C, S) -- and, amax, its largest magnitude into the
+// GEMM-side slot -- by the same launch)
+struct BiasJob {
+    const float *gout;
+    float *gb;
+    int B, C, S;
+    bool accumulate, amax;
+};
 hipError_t launch_to_channels_last(int dtype, const void *x, void *xcl, int B, int C, int Sn, hipStream_t s,
                                    int *flag = nullptr, const void *chk = nullptr, size_t chk_n = 0,
-                                   float chk_limit = 0.f, const void *amax_w = nullptr, size_t amax_w_n = 0);
+                                   float chk_limit = 0.f, const void *amax_w = nullptr, size_t amax_w_n = 0,
+                                   const BiasJob *bias = nullptr);
+// the copy's blocks per image, which a bias job's channels are dealt to
+inline long long copy_blocks(int C, int Sn) { return (long long)((Sn + 63) / 64) * ((C + 63) / 64); }
 // 16-bit MFMA operands of the sampled side (forward, weight gradient): the sampled values are
 // mask * bilinear(X), below 2^126 (finite, with a finite piece scale) when |X| < SAMPLED_LIMIT
 // and |mask| < MASK_LIMIT; larger or non-finite values send the launch to its fp32 MFMA loop.
