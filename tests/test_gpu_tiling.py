@@ -94,6 +94,19 @@ def test_half_layouts(case, dtype):
                     padding=[1] * dim, dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=90 + dim), dtype)
 
 
+# float32: the bias gradient beside the channels-last copy where that has a block for every other channel
+# (rows in whole quads and not, channels past the blocks, both directions), else a launch of its own
+BIAS = [(1, 144, 24, [304], False), (1, 144, 29, [301], False), (1, 144, 32, [301], False), (2, 68, 20, [16, 24], False),
+        (1, 32, 16, [300], True), (1, 32, 24, [300], True)]
+
+
+@pytest.mark.parametrize("case", BIAS, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
+def test_bias_gradient_launch(case):
+    dim, cin, cout, size, transposed = case
+    check(make_case(dim, transposed, batch=3, cin=cin, cout=cout, kernel=[3] * dim, stride=[1 + transposed] * dim,
+                    padding=[1] * dim, dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=95 + dim), torch.float32)
+
+
 # few sampled-side channels: column lengths (channels x taps) around the 16 and 64 blocks and at the rule's
 # ends, GEMM sides around 16 and 64, pixels around the 64 of a tile, more tiles than workgroups, offset and
 # mask groups that do not nest, conv groups, no offset / mask / bias
