@@ -146,7 +146,8 @@ tvdcn_status tvdcn_deform_conv_forward(const tvdcn_conv_desc *desc, const void *
  * copy of the input, the weight re-layout, the split accumulator) is a library-owned device array
  * of TVDCN_SCRATCH_BYTES per GPU, held until the process ends; its address is looked up at the
  * first call on each device. A problem whose forward workspace
- * (tvdcn_deform_conv_forward_workspace_size) exceeds TVDCN_SCRATCH_BYTES returns
+ * (tvdcn_deform_conv_forward_workspace_size) exceeds TVDCN_SCRATCH_BYTES even without partial sums
+ * (where only those exceed it, each output tile is summed by one workgroup) returns
  * TVDCN_STATUS_WORKSPACE_TOO_SMALL with a message naming both sizes (a float32 input passed
  * channels-last, TVDCN_FLAG_CHANNELS_LAST, needs no input copy: only the weight re-layout).
  * Every call on a GPU uses that GPU's one array: calls that overlap on one GPU (other streams,
