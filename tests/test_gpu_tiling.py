@@ -154,3 +154,25 @@ def test_few_channels_last(dtype):
     assert outs[1][1].is_contiguous(memory_format=torch.channels_last)
     for a, b in zip(*outs):
         assert rel_err(a, b) < (1e-6 if dtype == torch.float32 else 1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_data_gradient_in_several_launches(dtype):
+    """60000 images of 2 x 2 x 2 pixels in 24 groups, three passes of taps each: 4.32M workgroups of 1024 threads, more
+    than one launch takes. An image's gradients are those of a call on it alone: the first and the last ones, and
+    those on both sides of the second launch's first workgroup (72 an image)."""
+    batch, c, groups = 60000, 96, 24
+    g = torch.Generator(device="cuda").manual_seed(101)
+    rand = lambda *shape: torch.rand(*shape, generator=g, device="cuda").to(dtype)
+    x, w = rand(batch, c, 2, 2, 2), rand(c, c // groups, 3, 3, 3)
+    off, msk, gy = rand(batch, 81, 2, 2, 2), rand(batch, 27, 2, 2, 2), rand(batch, c, 2, 2, 2)
+    off = off * 4 - 2
+    backward = lambda s: torch.ops.tvdcn._deform_conv3d_backward(gy[s], x[s], w, off[s], msk[s], rand(c), [1] * 3, [1] * 3,
+                                                                 [1] * 3, groups)
+    full = backward(slice(None))
+    at = ((2 ** 32 - 1) // 1024 // 8 * 8) // 72
+    for lo in (0, at - 2, batch - 4):
+        part = backward(slice(lo, lo + 4))
+        for name, a, b in zip(("input", "offset", "mask"), (full[0], full[2], full[3]), (part[0], part[2], part[3])):
+            # (sums of at most 27 x 4 terms per value, in another order where atomics add them)
+            assert rel_err(a[lo:lo + 4], b) < (1e-5 if dtype == torch.float32 else 1e-2), (lo, name)

@@ -54,3 +54,49 @@ def test_transposed_layer_of_an_empty_input_is_refused(record, cin, dtype, batch
     r = record(problem(2, batch, cin, 4, [0, 4], [4, 4], transposed=True, padding=1, dtype=dtype))
     for call in r.values():
         assert call["status"] == INVALID_ARGUMENT and "positive" in call["error"] and not call["launches"]
+
+
+@pytest.mark.parametrize("cin", [3, 32])
+def test_layer_of_an_empty_input_is_refused(record, cin):
+    """Padding gives an empty input an output of 2 x 4 pixels: an error, few channels or many."""
+    r = record(problem(2, 2, cin, 32, [0, 4], [3, 3], padding=2))
+    for call in r.values():
+        assert call["status"] == INVALID_ARGUMENT and "positive" in call["error"] and not call["launches"]
+    assert record(problem(2, 0, cin, 32, [0, 4], [3, 3], padding=2))["forward"]["status"] == SUCCESS   # empty batch
+
+
+def blocks(call, kernel):
+    return [grid[0] for name, grid, _ in call["launches"] if kernel in name]
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("dim,batch,size,kernel,groups,tiles,threads", [
+    # 46M input values: 4.32M data gradient workgroups of 1024 threads, more than one launch takes
+    (3, 60000, [2, 2, 2], [3, 3, 3], 24, 60000 * 24 * 3, 1024),
+    (2, 2200000, [2, 1], [4, 4], 1, 2200000 * 6 * 2, 512)])
+def test_tiles_of_many_small_images(record, dim, batch, size, kernel, groups, tiles, threads, dtype):
+    """A tile per (image, 16-channel slice or group, pass of taps), however few its pixels, in one launch or two (the
+    scatter and the offset gradients)."""
+    r = record(problem(dim, batch, 96, 96, size, kernel, groups=groups, padding=1 if dim == 3 else 2, dtype=dtype, mg=0))
+    assert r["backward"]["status"] == SUCCESS, r["backward"]["error"]
+    runs = blocks(r["backward"], "bwd_data_win_kernel")
+    assert sum(runs) in (tiles, 2 * tiles) and max(runs) * threads < 2 ** 32
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_layouts_of_many_small_images(record, dtype, transposed):
+    """8388600 images of one pixel: a layout block of 256 threads for each of two operands, and others'."""
+    r = record(problem(1, 8388600, 16, 16, [1], [1], dtype=dtype, transposed=transposed))
+    for call in r.values():
+        assert call["status"] == SUCCESS, call["error"]
+    assert sum(blocks(r["backward"], "prep16_kernel")) > 2 ** 24
+
+
+@pytest.mark.parametrize("pixels", [2 ** 28 - 16, 2 ** 28, 2 ** 29 - 32])
+def test_few_channels_of_many_pixels(record, pixels):
+    """One channel of up to 2^31 - 128 positions: four threads per position below 2^30, the general kernels above."""
+    r = record(problem(1, 4, 1, 1, [pixels], [1], og=0, mg=0))
+    for call in r.values():
+        assert call["status"] == SUCCESS, call["error"]
+        assert bool(blocks(call, "few_")) == (4 * pixels < 2 ** 30)

@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(64 * NW)
 bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wchunks, const uint16_t *zs,
                     const uint16_t *wsplit, const int *flag, const float *__restrict__ xcl,
                     const T *__restrict__ offset, const T *__restrict__ mask, float *__restrict__ gx_cl,
-                    float *__restrict__ goff, float *__restrict__ gmask, const int gx_nchw) {
+                    float *__restrict__ goff, float *__restrict__ gmask, const int gx_nchw, const int first) {
     constexpr int NC = 1 << DIM;
     constexpr int TMAX = WIN_TMAX;
     constexpr int NT = 64 * NW;
@@ -191,7 +191,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     const int mq = 4 * q;
 
     // ---- tile: one spatial box x one 16-channel slice --------------------------------
-    int L = xcd_remap(blockIdx.x, gridDim.x);
+    int L = first + xcd_remap(blockIdx.x, gridDim.x);
     const int ct = L % wt.c_tiles;
     L /= wt.c_tiles;
     const int npass = (g.Kn + wt.tpp - 1) / wt.tpp;
@@ -1188,9 +1188,9 @@ __global__ void __launch_bounds__(256)
 data_prep_kernel(const T *__restrict__ z, uint16_t *__restrict__ zs, const T *__restrict__ w, uint16_t *__restrict__ wsp,
                  float *__restrict__ wd, int *flag, int G, int Mg, int Cg, int Pn, int Kn, int c_tiles, int ms32,
                  int m_steps, int pblocks, long long nz, int nws, bool zvec, uint16_t *__restrict__ zw,
-                 size_t zw_plane) {
+                 size_t zw_plane, const int first) {
     __shared__ float smem[WL_TK * BC * 33];
-    long long L = blockIdx.x;
+    long long L = first + (long long)blockIdx.x;
     if (L < nz) {
         z_split_block<T, NP>(L, smem, z, zs, zw, flag, G, Mg, Pn, ms32, pblocks, zvec, zw_plane);
         return;
@@ -1220,12 +1220,14 @@ hipError_t launch_w(const Geo &g, const WinTiles &tl, const void *z, const void 
     if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
         return e;
     const long long blocks = (long long)g.G * g.B * tl.ntile[0] * tl.ntile[1] * tl.ntile[2] * tl.c_tiles * ((g.Kn + tl.tpp - 1) / tl.tpp);
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * NW), lds, s, g, tl, static_cast<const T *>(z),
-                       static_cast<const float *>(wchunks), static_cast<const uint16_t *>(zs),
-                       static_cast<const uint16_t *>(wsplit), flag, static_cast<const float *>(xcl),
-                       static_cast<const T *>(offset), static_cast<const T *>(mask), static_cast<float *>(gx_cl),
-                       static_cast<float *>(goff), static_cast<float *>(gmask), gx_nchw ? 1 : 0);
-    return hipGetLastError();
+    if (blocks == 0) return hipErrorInvalidValue;
+    return launch_block_runs(blocks, 64 * NW, [&](int first, unsigned n) {
+        hipLaunchKernelGGL(kern, dim3(n), dim3(64 * NW), lds, s, g, tl, static_cast<const T *>(z),
+                           static_cast<const float *>(wchunks), static_cast<const uint16_t *>(zs),
+                           static_cast<const uint16_t *>(wsplit), flag, static_cast<const float *>(xcl),
+                           static_cast<const T *>(offset), static_cast<const T *>(mask), static_cast<float *>(gx_cl),
+                           static_cast<float *>(goff), static_cast<float *>(gmask), gx_nchw ? 1 : 0, first);
+    });
 }
 
 template <int DIM, typename T, bool SCATTER, bool COORD>
@@ -1286,15 +1288,15 @@ hipError_t launch_prep(const Geo &g, const WinTiles &t, const void *z, const voi
     const long long wblocks = (long long)g.G * t.c_tiles * t.ms32 * tchunks;
     const long long dblocks = wd != nullptr ? (long long)g.G * t.c_tiles * t.m_steps * tchunks : 0;
     const long long total = zblocks + wblocks + dblocks;
-    if (wblocks > INT_MAX || dblocks > INT_MAX || total > INT_MAX) return hipErrorInvalidValue;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL((data_prep_kernel<T, NP>), dim3((unsigned)total), dim3(256), 0, s, static_cast<const T *>(z),
-                       static_cast<uint16_t *>(zs), static_cast<const T *>(w), static_cast<uint16_t *>(wsp),
-                       static_cast<float *>(wd), flag, g.G, g.Mg, g.Cg, g.Pn, g.Kn, t.c_tiles, t.ms32, t.m_steps,
-                       pblocks, zblocks, (int)wblocks,
-                       g.Pn % 4 == 0 && reinterpret_cast<uintptr_t>(z) % (4 * sizeof(T)) == 0,
-                       static_cast<uint16_t *>(zw), (size_t)g.B * g.M * g.Pn);
-    return hipGetLastError();
+    if (wblocks > INT_MAX || dblocks > INT_MAX) return hipErrorInvalidValue;
+    return launch_block_runs(total, 256, [&](int first, unsigned n) {
+        hipLaunchKernelGGL((data_prep_kernel<T, NP>), dim3(n), dim3(256), 0, s, static_cast<const T *>(z),
+                           static_cast<uint16_t *>(zs), static_cast<const T *>(w), static_cast<uint16_t *>(wsp),
+                           static_cast<float *>(wd), flag, g.G, g.Mg, g.Cg, g.Pn, g.Kn, t.c_tiles, t.ms32, t.m_steps,
+                           pblocks, zblocks, (int)wblocks,
+                           g.Pn % 4 == 0 && reinterpret_cast<uintptr_t>(z) % (4 * sizeof(T)) == 0,
+                           static_cast<uint16_t *>(zw), (size_t)g.B * g.M * g.Pn, first);
+    });
 }
 
 int ilog2(int v) {

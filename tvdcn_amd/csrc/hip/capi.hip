@@ -142,8 +142,9 @@ tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch, bool l
         dl3[e] = d->dilation[i];
     }
     const int64_t Sn = S3[0] * S3[1] * S3[2], Pn = P3[0] * P3[1] * P3[2], Kn = K3[0] * K3[1] * K3[2];
-    // (a transposed layer may give an empty input a non-empty output; the pixel divisions need a column)
-    if (Pn <= 0) return fail(TVDCN_STATUS_INVALID_ARGUMENT, "the input's spatial size must be positive");
+    // (a kernel or its padding may give an empty input a non-empty output; the pixel divisions need a column,
+    // the kernels something to sample)
+    if (Pn <= 0 || (Sn <= 0 && batch > 0)) return fail(TVDCN_STATUS_INVALID_ARGUMENT, "the input's spatial size must be positive");
     const int64_t B = batch;
     // int32 indexing inside the kernels: every tensor of the block must stay below 2^31 elements
     const int64_t biggest[] = {B * C * Sn, B * M * Pn, M * (C / d->groups) * Kn,

@@ -343,8 +343,10 @@ FewPlan plan_few(const Geo &g, int dtype) {
     // 1535, 5 -> 512 k3 on 4 x 64x64 652 -> 280, 10 -> 512 666 -> 679, 14 -> 512 668 -> 882, 21 -> 30 on
     // 20x20 459 -> 214, 30 -> 30 on 16 x 128x128 4406 -> 9081). A fused mask
     // activation's gradient is finished in the accumulation type, which 16-bit gradients here never are.
+    // Fewer than 2^30 pixels: four threads each stay below HIP's 2^32 of a launch, and a run of tiles that
+    // ends past the last pixel below 2^31.
     const long long column = (long long)g.C * g.Kn;
-    f.ok = (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) && (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype) <= WIN_LDS_TARGET &&
+    f.ok = g.NP < 1 << 30 && (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) && (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype) <= WIN_LDS_TARGET &&
            (g.mask_act == 0 || dtype == kF32 || dtype == kF64);
     if (!f.ok || g.NP == 0) return f;
     const int tiles = (g.NP + BP - 1) / BP;

@@ -3,7 +3,9 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <atomic>
+#include <climits>
 #include "common.h"
 
 namespace tvdcn_hip {
@@ -48,6 +50,17 @@ inline hipError_t raise_lds_limit(const void *kern, std::atomic<unsigned long lo
     e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)WIN_LDS_TARGET);
     if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
     return e;
+}
+// launch(first, n) for each run of a grid's blocks: HIP takes fewer than 2^32 threads along x, so a grid of tiles
+// of many small images goes out in several launches. (Runs of a multiple of 8 blocks: even shares of the XCDs.)
+template <typename F> hipError_t launch_block_runs(long long blocks, int threads, F &&launch) {
+    if (blocks > INT_MAX) return hipErrorInvalidValue;   // the kernels count blocks in 32 bits
+    const long long run = 0xFFFFFFFFll / threads / 8 * 8;
+    for (long long first = 0; first < blocks; first += run) {
+        launch((int)first, (unsigned)std::min(run, blocks - first));
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 struct WinTiles {
     bool ok;             // eligible: fp32/fp16/bf16, C % 4 == 0, 16-channel tiles group-uniform

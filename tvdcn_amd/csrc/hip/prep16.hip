@@ -180,10 +180,10 @@ prep16_kernel(const Geo g, const Prep16Blocks nb, const Prep16Geo pg, const T *_
               const T *__restrict__ z, uint16_t *__restrict__ zs, uint16_t *__restrict__ zw, const T *__restrict__ w,
               uint16_t *__restrict__ wsp, uint16_t *__restrict__ w16, const int c_tiles, const int ms32, const int slices,
               const int nmb, const int tpp, const int hp, const int pp, const T *__restrict__ gout, T *__restrict__ gb,
-              float *__restrict__ f0, float *__restrict__ f1, float *__restrict__ f2) {
+              float *__restrict__ f0, float *__restrict__ f1, float *__restrict__ f2, const int first) {
     __shared__ __align__(16) float smem[WL_TK * BC * 33];
     static_assert(WL_TK * BC * 33 >= TT * (TT + 1), "the copy's tile");
-    unsigned L = blockIdx.x;
+    unsigned L = first + blockIdx.x;
     if (L < nb.cl) {
         if constexpr (V == 0) {
             widen_block<T>(L, x, xcl, pg.x_n);
@@ -227,9 +227,9 @@ __global__ void __launch_bounds__(256)
 out16_kernel(const float *__restrict__ acc, T *__restrict__ y, const T *__restrict__ bias, const int C, const int S,
              const int st, const int ct, const unsigned n_y, const float *__restrict__ a0, T *__restrict__ o0, const size_t n0,
              const unsigned nb0, const float *__restrict__ a1, T *__restrict__ o1, const size_t n1, const size_t ny,
-             const int vec) {
+             const int vec, const int first) {
     __shared__ __align__(16) float smem[TT * (TT + 1)];
-    unsigned L = blockIdx.x;
+    unsigned L = first + blockIdx.x;
     if (L < n_y) {
         if constexpr (V == 0) {
             narrow_block<T>(L, acc, y, ny, vec & 1);
@@ -324,18 +324,18 @@ hipError_t launch_prep16(int dtype, const Geo &g, const Prep16 &j, hipStream_t s
     // four 16-byte stores per thread on the largest accumulator
     if (most > 0) nb.fill = (unsigned)std::min<size_t>((most + 4095) / 4096, 4096);
     total += nb.fill;
-    if (total > INT_MAX) return hipErrorInvalidValue;
-    if (total == 0) return hipSuccess;
     auto go = [&](auto tv, auto vv) {
         using T = decltype(tv);
-        hipLaunchKernelGGL((prep16_kernel<T, decltype(vv)::value>), dim3((unsigned)total), dim3(256), 0, s, g, nb, pg,
-                           static_cast<const T *>(j.x), static_cast<float *>(j.xcl), static_cast<const T *>(j.z),
-                           static_cast<uint16_t *>(j.zs), static_cast<uint16_t *>(j.zw), static_cast<const T *>(j.w),
-                           static_cast<uint16_t *>(j.wsplit), static_cast<uint16_t *>(j.w16), j.wt ? j.wt->c_tiles : 0,
-                           j.wt ? j.wt->ms32 : 0, slices, j.fw ? j.fw->Mg_pad / 16 : 0, j.fw ? j.fw->tpp : 0,
-                           j.fw ? j.fw->hp : 0, j.fw ? j.fw->pp : 0, static_cast<const T *>(j.gout), static_cast<T *>(j.gb),
-                           static_cast<float *>(j.fill[0]), static_cast<float *>(j.fill[1]), static_cast<float *>(j.fill[2]));
-        return hipGetLastError();
+        return launch_block_runs(total, 256, [&](int first, unsigned n) {
+            hipLaunchKernelGGL((prep16_kernel<T, decltype(vv)::value>), dim3(n), dim3(256), 0, s, g, nb, pg,
+                               static_cast<const T *>(j.x), static_cast<float *>(j.xcl), static_cast<const T *>(j.z),
+                               static_cast<uint16_t *>(j.zs), static_cast<uint16_t *>(j.zw), static_cast<const T *>(j.w),
+                               static_cast<uint16_t *>(j.wsplit), static_cast<uint16_t *>(j.w16), j.wt ? j.wt->c_tiles : 0,
+                               j.wt ? j.wt->ms32 : 0, slices, j.fw ? j.fw->Mg_pad / 16 : 0, j.fw ? j.fw->tpp : 0,
+                               j.fw ? j.fw->hp : 0, j.fw ? j.fw->pp : 0, static_cast<const T *>(j.gout),
+                               static_cast<T *>(j.gb), static_cast<float *>(j.fill[0]), static_cast<float *>(j.fill[1]),
+                               static_cast<float *>(j.fill[2]), first);
+        });
     };
     switch (dtype) {
         case kF16: return by_vec<__half>(v, go);
@@ -351,16 +351,15 @@ hipError_t launch_out16(int dtype, const Out16 &j, hipStream_t s) {
     const long long n_y = j.acc == nullptr ? 0 : j.cl ? flat_blocks(ny) : (long long)st * ct * j.B;
     const unsigned nb0 = j.a0 != nullptr ? flat_blocks(j.n0) : 0, nb1 = j.a1 != nullptr ? flat_blocks(j.n1) : 0;
     const long long total = n_y + nb0 + nb1;
-    if (total > INT_MAX) return hipErrorInvalidValue;
-    if (total == 0) return hipSuccess;
     const int vec = (aligned_to(j.y, 8) ? 1 : 0) | (aligned_to(j.o0, 8) ? 2 : 0) | (aligned_to(j.o1, 8) ? 4 : 0);
     auto go = [&](auto tv, auto vv) {
         using T = decltype(tv);
-        hipLaunchKernelGGL((out16_kernel<T, decltype(vv)::value>), dim3((unsigned)total), dim3(256), 0, s,
-                           static_cast<const float *>(j.acc), static_cast<T *>(j.y), static_cast<const T *>(j.bias), j.C, j.S,
-                           st, ct, (unsigned)n_y, static_cast<const float *>(j.a0), static_cast<T *>(j.o0), j.n0, nb0,
-                           static_cast<const float *>(j.a1), static_cast<T *>(j.o1), j.n1, ny, vec);
-        return hipGetLastError();
+        return launch_block_runs(total, 256, [&](int first, unsigned n) {
+            hipLaunchKernelGGL((out16_kernel<T, decltype(vv)::value>), dim3(n), dim3(256), 0, s,
+                               static_cast<const float *>(j.acc), static_cast<T *>(j.y), static_cast<const T *>(j.bias), j.C,
+                               j.S, st, ct, (unsigned)n_y, static_cast<const float *>(j.a0), static_cast<T *>(j.o0), j.n0, nb0,
+                               static_cast<const float *>(j.a1), static_cast<T *>(j.o1), j.n1, ny, vec, first);
+        });
     };
     switch (dtype) {
         case kF16: return by_vec<__half>(v, go);
