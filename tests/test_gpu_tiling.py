@@ -97,7 +97,7 @@ def test_half_layouts(case, dtype):
 # float32: the bias gradient beside the channels-last copy where that has a block for every other channel
 # (rows in whole quads and not, channels past the blocks, both directions), else a launch of its own
 BIAS = [(1, 144, 24, [304], False), (1, 144, 29, [301], False), (1, 144, 32, [301], False), (2, 68, 20, [16, 24], False),
-        (1, 32, 16, [300], True), (1, 32, 24, [300], True)]
+        (1, 32, 16, [300], True), (1, 32, 24, [300], True), (1, 16, 20, [4097], False), (1, 16, 20, [8191], False)]
 
 
 @pytest.mark.parametrize("case", BIAS, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
