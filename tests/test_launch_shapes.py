@@ -100,3 +100,15 @@ def test_few_channels_of_many_pixels(record, pixels):
     for call in r.values():
         assert call["status"] == SUCCESS, call["error"]
         assert bool(blocks(call, "few_")) == (4 * pixels < 2 ** 30)
+
+
+@pytest.mark.parametrize("dim,size,kernel,channels,few", [
+    (1, [5000], [13], 9, True), (1, [5041], [13], 9, True), (1, [5042], [13], 9, False), (1, [90000], [13], 5, True),
+    (2, [64, 64], [4, 4], 3, True), (2, [64, 65], [4, 4], 3, False), (2, [8, 8], [4, 4], 5, False),
+    (2, [300, 300], [4, 4], 2, True), (3, [3, 4, 4], [3, 3, 3], 2, False), (3, [40, 40, 40], [4, 4, 4], 1, True)])
+def test_transposed_forward_of_few_channels(record, dim, size, kernel, channels, few):
+    """The scatter of the few-channel kernels costs a cache line per (pixel, channel): the general kernels' for more
+    channels, on larger grids and in higher rank. The backward, whose weight gradient counts too, stays few."""
+    r = record(problem(dim, 1, 16, channels, size, kernel, transposed=True, stride=2, padding=1))
+    assert bool(blocks(r["forward"], "few_")) == few and bool(blocks(r["forward"], "bwd_data_kernel")) == (not few)
+    assert bool(blocks(r["backward"], "few_data_kernel"))

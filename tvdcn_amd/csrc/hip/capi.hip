@@ -211,8 +211,8 @@ tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch, bool l
                                x_window_cell_bytes());
     pl.ww = plan_weight_win(g, pl.wn_w, pl.dim);
     pl.fw = plan_fwd_win(g, pl.wn_s, pl.dim, pl.wn_f, lean);
-    pl.few = plan_few(g, pl.dtype);
-    if (pl.wn_s.ok) pl.few.ok = false;
+    pl.few = plan_few(g, pl.dtype, pl.dim);
+    if (pl.wn_s.ok) pl.few.ok = pl.few.scatter = false;
     const bool cl_in = (d->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
     // (1D only: there a window row is the tile's 256 pixels + margins, whole lines of each channel;
     // 2D / 3D window rows are 10-26 cells, and the flush and out-of-window corners then reach
@@ -323,7 +323,7 @@ Layout layout(const Plan &pl, bool backward) {
     L.xcl = L.wf = L.wd = L.cl_acc = L.wpart = L.goff_acc = L.gmask_acc = L.yacc = SENTINEL;
     L.zs = L.wsplit = L.w16 = L.flag = L.zw = SENTINEL;
     L.flag = take(align_up(sizeof(int) * OPERAND_FLAG_WORDS));   // the flag and the operands' largest magnitudes
-    if (pl.few.ok) {
+    if (backward || !pl.transposed ? pl.few.ok : pl.few.scatter) {
         // the input gradient / transposed output in the accumulation type, the weight gradient's sums
         if (!acc_is_storage(pl.dtype) && backward != pl.transposed) L.cl_acc = take(cl_bytes);
         if (backward) L.wpart = take(align_up(pl.few.part_elems * a));
@@ -562,7 +562,7 @@ tvdcn_status forward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const 
     const int dt = pl.dtype;
     g_last_error.clear();
     int *flag = static_cast<int *>(at(workspace, L.flag));
-    if (pl.few.ok) {
+    if (pl.transposed ? pl.few.scatter : pl.few.ok) {
         const bool cl = (desc->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
         if (!pl.transposed) {
             TVDCN_LAUNCH(TVDCN_KERNEL_GATHER_GEMM, s,

@@ -329,16 +329,16 @@ template <typename F> hipError_t by_type(int dtype, int dim, F &&f) {
 
 size_t acc_bytes(int dtype) { return dtype == kF64 ? sizeof(double) : sizeof(float); }
 size_t fwd_lds(const Geo &g, int dtype) { return (size_t)g.C * g.Kn * LDF * acc_bytes(dtype); }
-size_t data_lds(const Geo &g, int dtype) {
-    return (size_t)(2 * g.C * g.Kn + 1) * LDG * acc_bytes(dtype) + BP * sizeof(int);
+// (weight: the columns beside G, for the weight gradient)
+size_t data_lds(const Geo &g, int dtype, bool weight) {
+    return (size_t)((weight ? 2 : 1) * g.C * g.Kn + (weight ? 1 : 0)) * LDG * acc_bytes(dtype) + BP * sizeof(int);
 }
 
 }  // namespace
 
-FewPlan plan_few(const Geo &g, int dtype) {
+FewPlan plan_few(const Geo &g, int dtype, int dim) {
     FewPlan f{};
-    // Columns of up to 128 values (G and S of a tile leave room for two workgroups per CU in fp32), or 200
-    // on grids of up to a tile per CU, and weights of up to 24576: beyond either the general kernels'
+    // Columns of up to 128 values, or 200 on grids of up to a tile per CU, and weights of up to 24576: beyond either the general kernels'
     // wider tiles win (float32, us a training step, general -> here: 3 -> 64 k3 on 8 x 224x224 5476 ->
     // 1535, 5 -> 512 k3 on 4 x 64x64 652 -> 280, 10 -> 512 666 -> 679, 14 -> 512 668 -> 882, 21 -> 30 on
     // 20x20 459 -> 214, 30 -> 30 on 16 x 128x128 4406 -> 9081). A fused mask
@@ -346,9 +346,18 @@ FewPlan plan_few(const Geo &g, int dtype) {
     // Fewer than 2^30 pixels: four threads each stay below HIP's 2^32 of a launch, and a run of tiles that
     // ends past the last pixel below 2^31.
     const long long column = (long long)g.C * g.Kn;
-    f.ok = g.NP < 1 << 30 && (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) && (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype) <= WIN_LDS_TARGET &&
+    f.ok = g.NP < 1 << 30 && (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) && (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype, true) <= WIN_LDS_TARGET &&
            (g.mask_act == 0 || dtype == kF32 || dtype == kF64);
     if (!f.ok || g.NP == 0) return f;
+    // The scatter alone (the transposed forward): a lane per pixel, so that an atomic instruction reaches up to 64
+    // lines for one channel, where the general kernel's covers the channels of a pixel's corner, one line. Its cost
+    // grows with the channels, the general kernel's hardly. float32, us a call, general -> here: 1D k16 on
+    // 8 x 65536, 3 / 5 / 7 channels 1591 -> 928, 1542 -> 1506, 1594 -> 2087; 2D k4 on 8 x 128x128, 1 / 2 / 3
+    // channels 649 -> 280, 595 -> 548, 655 -> 835; 3D k4 on 2 x 8x28x28, 1 / 2 channels 399 -> 250, 366 -> 486.
+    // Small layers have a launch less here: 1D k3 on 4 x 4096, 9 channels 30 -> 22, 2D k4 on 2 x 32x32, 3 / 5
+    // channels 33 -> 28, 33 -> 43.
+    const bool small = (long long)g.NP * g.Kn <= 65536;
+    f.scatter = g.C <= (dim == 1 ? (small ? 9 : 5) : dim == 2 ? (small ? 3 : 2) : 1);
     const int tiles = (g.NP + BP - 1) / BP;
     // one tile per workgroup up to one per CU, then runs of tiles (each workgroup's partial sums of dW are
     // read back by the reduction)
@@ -389,11 +398,16 @@ hipError_t launch_few_data(int dtype, int dim, const Geo &g, const FewPlan &f, c
         static std::atomic<unsigned long long> lds_raised{0};
         const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3((unsigned)f.splits), dim3(64 * NW), data_lds(g, dtype), s, g,
+        // without a weight gradient (the transposed forward) there are no partial sums to read back, and a tile needs
+        // half the LDS: a workgroup per tile, as many on a CU as fit (64 -> 1 channel k4 on 8 x 128x128 294 -> 285 us
+        // against runs of tiles, 1D k16 on 8 x 65536 542 -> 509)
+        const bool weight = part != nullptr;
+        const int tiles = (g.NP + BP - 1) / BP;
+        hipLaunchKernelGGL(kern, dim3((unsigned)(weight ? f.splits : tiles)), dim3(64 * NW), data_lds(g, dtype, weight), s, g,
                            static_cast<const T *>(z), static_cast<const T *>(x), x_cl ? 1 : g.Sn, x_cl ? g.C : 1,
                            static_cast<const T *>(w), static_cast<const T *>(offset), static_cast<const T *>(mask),
                            static_cast<A *>(gx), static_cast<T *>(goff), static_cast<T *>(gmask), static_cast<A *>(part),
-                           f.chunks);
+                           weight ? f.chunks : 1);
         return hipGetLastError();
     });
 }

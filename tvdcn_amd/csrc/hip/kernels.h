@@ -126,13 +126,14 @@ struct FwdWin {
 // Layers of few sampled-side channels (few_channels.hip): the columns of 64-pixel tiles whole in LDS
 struct FewPlan {
     bool ok;             // a pixel's column, C * Kn values, fits (and any mask activation is finished in fp32 / fp64)
+    bool scatter;        // ok, and the transposed forward too
     int chunks;          // 64-pixel tiles per workgroup of the data kernel
     int splits;          // its workgroups
     size_t part_elems;   // accumulator elements of their weight / bias gradient sums: [splits][M][Cg * Kn + 1]
 };
 
 FwdTiles plan_fwd(const Geo &g, int dtype);
-FewPlan plan_few(const Geo &g, int dtype);
+FewPlan plan_few(const Geo &g, int dtype, int dim);
 // windowed forward plan over the base tiling; wt receives the tiling with the forward's
 // own window margin (lean: one share per tile, so no partials in the workspace)
 FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, bool lean = false);
