@@ -176,3 +176,17 @@ def test_data_gradient_in_several_launches(dtype):
         for name, a, b in zip(("input", "offset", "mask"), (full[0], full[2], full[3]), (part[0], part[2], part[3])):
             # (sums of at most 27 x 4 terms per value, in another order where atomics add them)
             assert rel_err(a[lo:lo + 4], b) < (1e-5 if dtype == torch.float32 else 1e-2), (lo, name)
+
+
+def test_few_channels_bias_gradient_of_equal_values():
+    """The bias gradient of few channels over 100352 equal values a channel, which leave the roundings of a chain of
+    additions on one side: 6 levels of a tree over 64 lanes, 7 tiles' sums a workgroup, 7 + 2 + 3 additions of 224
+    workgroups' sums. At most 25 roundings of 2^-24 of the sum so far."""
+    values = torch.linspace(0.1, 1.3, 24, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(102)
+    rand = lambda *shape: torch.rand(*shape, generator=g, device="cuda")
+    gy = values.reshape(1, 24, 1, 1).expand(8, 24, 112, 112).contiguous()
+    gb = torch.ops.tvdcn._deform_conv2d_backward(gy, rand(8, 3, 112, 112), rand(24, 3, 1, 1), rand(8, 2, 112, 112),
+                                                 rand(8, 1, 112, 112), rand(24), [1, 1], [0, 0], [1, 1], 1)[4]
+    exact = values.double() * 8 * 112 * 112
+    assert float(((gb.double() - exact) / exact).abs().max()) < 25 * 2.0 ** -24

@@ -5,7 +5,7 @@
 //   forward (and the transposed op's grad_input): Y[m][p] = bias[m] + sum_k W[m][k] S[k][p]
 //   data: G[k][p] = sum_m W[m][k] Z[m][p], then per (pixel, tap) the scatter of mask * G into dX, the
 //         offset / mask gradients (a thread holds every channel of its pixel and tap: plain stores, no
-//         accumulators), and dW[m][k] (with the bias gradient as one more column, S = 1) = sum_p Z S
+//         accumulators), dW[m][k] = sum_p Z S, and the bias gradient sum_p Z
 //
 // Replaces the same reference pairs as the general kernels (tvdcn/csrc/ops/cuda/
 // deform_conv2d_kernel.cpp:341-380, 518-626 and the 1D / 3D twins). These calls are a few microseconds
@@ -26,6 +26,27 @@ constexpr int NW = 4;     // waves: 16 pixels each in the contractions, every fo
 // LDS row strides: 16 lanes along a row and 4 rows (forward), or 16 rows and 4 along a row (weight
 // gradient) fall on different banks
 constexpr int LDF = BP + 16, LDG = BP + 4;
+
+// Sum over the wave, in every lane: a tree (fp32 on the VALU: quad xor 1, quad xor 2, half-row mirror, row mirror,
+// then the rows swapped; fp64 through the LDS crossbar)
+__device__ __forceinline__ float wave_sum(float v) {
+    auto dpp = [&](auto ctrl) {
+        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    dpp(std::integral_constant<int, 0xB1>());
+    dpp(std::integral_constant<int, 0x4E>());
+    dpp(std::integral_constant<int, 0x141>());
+    dpp(std::integral_constant<int, 0x140>());
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
 
 // The corners of one (pixel, tap, offset group)
 template <int DIM, typename A> struct CornerSet {
@@ -141,8 +162,8 @@ few_data_kernel(const Geo g, const T *__restrict__ z, const T *__restrict__ x, c
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int K = g.C * g.Kn, Kg = g.Cg * g.Kn;
     A *Gs = reinterpret_cast<A *>(smem_raw);      // [K][LDG]
-    A *S = Gs + (size_t)K * LDG;                  // [K + 1][LDG], the last row ones (part)
-    int *zo = reinterpret_cast<int *>(S + (part != nullptr ? (size_t)(K + 1) * LDG : 0));   // [BP] offsets of the pixels in z
+    A *S = Gs + (size_t)K * LDG;                  // [K][LDG] (part)
+    int *zo = reinterpret_cast<int *>(S + (part != nullptr ? (size_t)K * LDG : 0));   // [BP] offsets of the pixels in z
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4;
     const A zero = A(0);
     const bool coord = goff != nullptr || gmask != nullptr;
@@ -244,22 +265,38 @@ few_data_kernel(const Geo g, const T *__restrict__ z, const T *__restrict__ x, c
             });
         }
         if (part != nullptr) {
-            if (wave == 0) S[K * LDG + lane] = ok ? A(1) : zero;
             __syncthreads();
-            // ---- dW[m][k], k = Kg the bias gradient: 16 x 16 blocks dealt to the waves; each is added to
-            //      the workgroup's partial sums of its earlier tiles
-            const int mb = (g.Mg + 15) / 16, kb = (Kg + 16) / 16;
+            // ---- bias gradient: the tile's sum of a row of Z by a tree over the lanes, then the tiles in turn (a column
+            //      of ones beside dW's had a chain of all the workgroup's pixels: error 7.4e-7 on 8 x 224x224, 1.5e-7
+            //      so). Lane i keeps row i of the wave's 64, so that a tile reads and writes its partial sums once.
+            for (int m0 = 0; m0 < g.M; m0 += 64 * NW) {
+                const int ml = m0 + wave + NW * lane;
+                A *dst = part + (size_t)ml * (Kg + 1) + Kg;
+                const A before = ch > 0 && ml < g.M ? *dst : zero;
+                const int rows = min(64, (g.M - m0 - wave + NW - 1) / NW);
+                const T *zr = z + (size_t)b * g.M * g.Pn + (size_t)(m0 + wave) * g.Pn + p;
+                A sum = zero;
+#pragma unroll 8
+                for (int i = 0; i < rows; ++i) {
+                    const A v = wave_sum(ok ? to_acc<A>(zr[(size_t)i * NW * g.Pn]) : zero);
+                    sum = lane == i ? v : sum;
+                }
+                if (ml < g.M) *dst = before + sum;
+            }
+            // ---- dW[m][k]: 16 x 16 blocks dealt to the waves; each is added to the workgroup's partial sums of its
+            //      earlier tiles
+            const int mb = (g.Mg + 15) / 16, kb = (Kg + 15) / 16;
             for (int i = wave; i < g.G * mb * kb; i += NW) {
                 const int k = i % kb * 16 + (lane & 15), r = i / kb;
                 const int m0 = r % mb * 16, grp = r / mb;
                 const int m = min(m0 + (lane & 15), g.Mg - 1);   // (rows past Mg: not stored)
                 const T *zr = z + ((size_t)grp * g.Mg + m) * g.Pn;
-                const A *Sr = S + (size_t)(k < Kg ? grp * Kg + k : K) * LDG;
+                const A *Sr = S + (size_t)(grp * Kg + min(k, Kg - 1)) * LDG;   // (columns past Kg: not stored)
                 acc4 acc;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int mr = m0 + mfma_row<A>(lane, v);
-                    acc[v] = ch > 0 && mr < g.Mg && k <= Kg ? part[((size_t)grp * g.Mg + mr) * (Kg + 1) + k] : zero;
+                    acc[v] = ch > 0 && mr < g.Mg && k < Kg ? part[((size_t)grp * g.Mg + mr) * (Kg + 1) + k] : zero;
                 }
 #pragma unroll
                 for (int s = 0; s < BP; s += 4) {
@@ -269,7 +306,7 @@ few_data_kernel(const Geo g, const T *__restrict__ z, const T *__restrict__ x, c
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int mr = m0 + mfma_row<A>(lane, v);
-                    if (mr < g.Mg && k <= Kg) part[((size_t)grp * g.Mg + mr) * (Kg + 1) + k] = acc[v];
+                    if (mr < g.Mg && k < Kg) part[((size_t)grp * g.Mg + mr) * (Kg + 1) + k] = acc[v];
                 }
             }
         }
@@ -278,24 +315,29 @@ few_data_kernel(const Geo g, const T *__restrict__ z, const T *__restrict__ x, c
 }
 
 // gw[m][k] = (accumulate: gw +) sum over the splits of part[split][m][k], gbias[m] the same of column Kg.
-// Block = 32 columns x 8 runs of splits, the runs' sums added in order.
+// Block = 32 columns x 8 runs of splits, four sums each; added in a fixed tree.
 template <typename T, typename A>
 __global__ void __launch_bounds__(256) few_reduce_kernel(const A *__restrict__ part, T *__restrict__ gw, T *__restrict__ gb,
                                                          int M, int Kg, int splits, bool accumulate) {
     __shared__ A sums[8][32];
     const int e = blockIdx.x * 32 + (threadIdx.x & 31), r = threadIdx.x >> 5;
     const int n = M * (Kg + 1);
-    A v = A(0);
+    A a[4] = {A(0), A(0), A(0), A(0)};
     if (e < n) {
         const int per = (splits + 7) / 8, s1 = min(splits, (r + 1) * per);
-#pragma unroll 8
-        for (int s = r * per; s < s1; ++s) v += part[(size_t)s * n + e];
+        int s = r * per;
+        for (; s + 8 <= s1; s += 8)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[i % 4] += part[(size_t)(s + i) * n + e];
+#pragma unroll
+        for (int i = 0; i < 7; ++i)
+            if (s + i < s1) a[i % 4] += part[(size_t)(s + i) * n + e];
     }
-    sums[r][threadIdx.x & 31] = v;
+    sums[r][threadIdx.x & 31] = (a[0] + a[1]) + (a[2] + a[3]);
     __syncthreads();
     if (r != 0 || e >= n) return;
-#pragma unroll
-    for (int i = 1; i < 8; ++i) v += sums[i][threadIdx.x];
+    auto at = [&](int i) { return sums[i][threadIdx.x]; };
+    const A v = ((at(0) + at(1)) + (at(2) + at(3))) + ((at(4) + at(5)) + (at(6) + at(7)));
     const int m = e / (Kg + 1), k = e - m * (Kg + 1);
     if (k == Kg && gb == nullptr) return;
     T *dst = k < Kg ? gw + (size_t)m * Kg + k : gb + m;
@@ -331,7 +373,7 @@ size_t acc_bytes(int dtype) { return dtype == kF64 ? sizeof(double) : sizeof(flo
 size_t fwd_lds(const Geo &g, int dtype) { return (size_t)g.C * g.Kn * LDF * acc_bytes(dtype); }
 // (weight: the columns beside G, for the weight gradient)
 size_t data_lds(const Geo &g, int dtype, bool weight) {
-    return (size_t)((weight ? 2 : 1) * g.C * g.Kn + (weight ? 1 : 0)) * LDG * acc_bytes(dtype) + BP * sizeof(int);
+    return (size_t)(weight ? 2 : 1) * g.C * g.Kn * LDG * acc_bytes(dtype) + BP * sizeof(int);
 }
 
 }  // namespace
