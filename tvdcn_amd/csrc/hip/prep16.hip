@@ -135,24 +135,33 @@ __device__ __forceinline__ void narrow_block(unsigned block, const float *__rest
     }
 }
 
-// grad_bias of channel c, the block's 256 threads over batch and space (vec: rows of whole aligned quads);
-// per-thread sums in a fixed order, then a fixed tree
+// grad_bias of channel c, the block's 256 threads over batch and space (vec: rows of whole aligned quads): four
+// sums per thread and row in a fixed order, then a fixed tree (one sum per thread was a chain four times as long
+// as the 1024 threads of a launch of its own have)
 template <typename T>
 __device__ __forceinline__ void bias_block(float *smem, const T *__restrict__ gout, T *__restrict__ gb, int c, int B, int C,
                                            int S, bool vec, bool accumulate) {
     float acc = 0.f;
     for (int b = 0; b < B; ++b) {
         const T *row = gout + ((size_t)b * C + c) * S;
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
         if (vec) {
 #pragma unroll 4
             for (int s = 4 * threadIdx.x; s < S; s += 1024) {
                 const Vec4<float> v = load4_t<float, T>(row + s);
-                acc += (v.x + v.y) + (v.z + v.w);
+                a[0] += v.x, a[1] += v.y, a[2] += v.z, a[3] += v.w;
             }
         } else {
-#pragma unroll 4
-            for (int s = threadIdx.x; s < S; s += 256) acc += to_acc<float>(row[s]);
+            // (every load unconditional, past the row's end its last value: one under a condition is waited for alone)
+            for (int s0 = threadIdx.x; s0 < S; s0 += 4096) {
+                float v[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) v[k] = to_acc<float>(row[min(s0 + 256 * k, S - 1)]);
+#pragma unroll
+                for (int k = 0; k < 16; ++k) a[k % 4] += s0 + 256 * k < S ? v[k] : 0.f;
+            }
         }
+        acc += (a[0] + a[1]) + (a[2] + a[3]);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
