@@ -190,3 +190,19 @@ def test_few_channels_bias_gradient_of_equal_values():
                                                  rand(8, 1, 112, 112), rand(24), [1, 1], [0, 0], [1, 1], 1)[4]
     exact = values.double() * 8 * 112 * 112
     assert float(((gb.double() - exact) / exact).abs().max()) < 25 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dim,batch,cin,size,kernel", [
+    (1, 3, 48, [300], 3), (2, 3, 32, [20, 24], 3), (2, 17, 160, [64, 64], 3), (3, 2, 16, [4, 5, 6], 1),
+    (3, 3, 32, [8, 16, 16], 3)], ids=lambda v: str(v).replace(" ", ""))
+def test_forward_loops(dim, batch, cin, size, kernel):
+    """One sampled value of the first image too large for the scaled 16-bit pieces sends the launch to the float32 loop,
+    in the same kernel or one of its own: the other images' results are those of the 16-bit loop, both within the
+    parity tests' float32 bound of the exact ones."""
+    case = make_case(dim, batch=batch, cin=cin, cout=20, kernel=[kernel] * dim, stride=[1] * dim,
+                     padding=[kernel // 2] * dim, dilation=[1] * dim, in_size=size, seed=110 + dim + batch)
+    x, w, off, msk, b = (case[n].to("cuda", torch.float32) for n in ("input", "weight", "offset", "mask", "bias"))
+    op = getattr(tvdcn, f"deform_conv{dim}d")
+    y = op(x, w, off, msk, b, padding=kernel // 2)
+    x[0].view(-1)[0] = 2.0 ** 127
+    assert rel_err(op(x, w, off, msk, b, padding=kernel // 2)[1:], y[1:]) < 2e-5

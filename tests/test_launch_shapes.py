@@ -112,3 +112,13 @@ def test_transposed_forward_of_few_channels(record, dim, size, kernel, channels,
     r = record(problem(dim, 1, 16, channels, size, kernel, transposed=True, stride=2, padding=1))
     assert bool(blocks(r["forward"], "few_")) == few and bool(blocks(r["forward"], "bwd_data_kernel")) == (not few)
     assert bool(blocks(r["backward"], "few_data_kernel"))
+
+
+@pytest.mark.parametrize("dim,batch,channels,size,kernel,launches", [
+    (1, 1, 16, [100], 3, 1), (1, 16, 512, [4096], 5, 1), (2, 1, 16, [8, 8], 1, 1), (2, 2, 256, [64, 64], 3, 1),
+    (2, 8, 256, [64, 64], 3, 2), (3, 1, 16, [4, 4, 4], 1, 1), (3, 2, 64, [16, 56, 56], 3, 2)])
+def test_float32_forward_loops(record, dim, batch, channels, size, kernel, launches):
+    """The float32 forward's two loops, of which a flag on the device selects one: two kernels where that is faster
+    than one kernel of both, whose launch that is not selected costs 4 us."""
+    r = record(problem(dim, batch, channels, channels, size, [kernel] * dim, padding=kernel // 2))
+    assert len(blocks(r["forward"], "fwd_win_kernel")) == launches

@@ -77,14 +77,15 @@ __device__ __forceinline__ void store_frag(const Geo &g, T *yg, int m0, int p, b
     }
 }
 
-// STAGE: the 16-bit loop's weight blocks are staged in LDS (1D / 2D, fw.stage_bytes > 0). USE16: the 16x16x32
-// MFMA loop; an fp32 call launches both instantiations and the operand flag has one return at once. ONE: a
-// single pass of taps. Either loop beside the other, or beside a loop over the passes, cost the 2D kernel 75
-// registers and 226 spilled scalars (174 and none without), the compiler keeping both loops' and all phases'
-// values live. (always_inline: at this size
-// the inliner otherwise leaves the lambdas as calls.) us a call: 256 channels, k3, 8 x 64x64, float32 training
-// 843 -> 839, bfloat16 128 channels, 2 x 100x152 inference 107 -> 103.
-template <int DIM, typename T, int MB, bool STAGE, bool USE16, bool ONE>
+// STAGE: the 16-bit loop's weight blocks are staged in LDS (1D / 2D, fw.stage_bytes > 0). LOOP: the 16x16x32 MFMA
+// loop, the fp32 one, or both, of which the operand flag selects one. ONE: a single pass of taps. Either loop
+// beside the other, or beside a loop over the passes, cost the 2D kernel 75 registers and 226 spilled scalars (174
+// and none without), the compiler keeping both loops' and all phases' values live. fp16 / bf16 run the 16-bit
+// loop alone; a long fp32 call launches either loop's kernel and the flag has one return at once, a short one both
+// in one kernel (launch_k). (always_inline: at this size the inliner otherwise leaves the lambdas as calls.)
+// bfloat16 128 channels, 2 x 100x152 inference 107 -> 103 us.
+constexpr int LOOP_F32 = 0, LOOP_16 = 1, LOOP_BOTH = 2;
+template <int DIM, typename T, int MB, bool STAGE, int LOOP, bool ONE>
 __global__ void __launch_bounds__(NT)
 fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__restrict__ xcl,
                const float *__restrict__ wf, const uint16_t *__restrict__ w16, const int *flag,
@@ -112,10 +113,12 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
     const int grp = L / n_sp;
     const bool deformable = offset != nullptr;
     const int slices = (g.Cg + BC - 1) / BC;
-    if (npiece_of<T>() == 2 && flag != nullptr && (*flag == 0) != USE16) return;   // the other launch's
+    const bool flagged = npiece_of<T>() == 2 && flag != nullptr && *flag != 0;
+    if (LOOP != LOOP_BOTH && npiece_of<T>() == 2 && flag != nullptr && flagged != (LOOP == LOOP_F32)) return;   // the other launch's
+    const bool use16 = LOOP == LOOP_16 || (LOOP == LOOP_BOTH && w16 != nullptr && !flagged);
     // fp32 as fp16 pieces: the sampled columns' scale, and the one back out (the weight's with it)
-    const int s_b = npiece_of<T>() == 2 && USE16 ? sampled_scale(g, flag, mask != nullptr) : 0;
-    const int s_back = npiece_of<T>() == 2 && USE16 ? -(s_b + operand_scale(flag, AMAX_W)) : 0;
+    const int s_b = npiece_of<T>() == 2 && use16 ? sampled_scale(g, flag, mask != nullptr) : 0;
+    const int s_back = npiece_of<T>() == 2 && use16 ? -(s_b + operand_scale(flag, AMAX_W)) : 0;
     // the sampling table's masks carry 2^s_b, so that the B fragments come out of the sampling at
     // their pieces' scale
     const float mscale_b = ldexpf(1.f, s_b);
@@ -468,7 +471,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 for (int j = 0; j < 4; ++j) bq[j][pb] = sv[j];
             }
         };
-        if constexpr (USE16) {
+        if (use16) {
             // 16x16x32 steps: a group's four taps are two tap pairs, each pair's B fragment its
             // two sampled quads (the 16-bit loop's K order, W16 below), split into pieces (fp32)
             // or rounded to T; the pair's A fragments come from global memory, each row block's
@@ -579,7 +582,7 @@ fwd_win_kernel(const Geo g, const WinTiles wt, const FwdWin fw, const float *__r
                 }
             });
         }
-    } else if constexpr (USE16) {
+    } else if (use16) {
         passes(pass16);
     } else {
         passes([&](int t0, int ntaps) __attribute__((always_inline)) {
@@ -715,11 +718,11 @@ fwd_w16_kernel(const T *__restrict__ w, uint16_t *__restrict__ out, int *flag, i
     w16_block<T, NP>(blockIdx.x, gridDim.x, w, out, flag, G, Mg, Cg, Kn, slices, nmb, tpp, hp, pp);
 }
 
-template <int DIM, typename T, int MB, bool STAGE, bool USE16, bool ONE>
+template <int DIM, typename T, int MB, bool STAGE, int LOOP, bool ONE>
 hipError_t launch_k1(const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl, const void *wf,
                     const void *w16, const int *flag, const void *offset, const void *mask, const void *bias, void *y,
                     void *y32, hipStream_t s) {
-    auto kern = fwd_win_kernel<DIM, T, MB, STAGE, USE16, ONE>;
+    auto kern = fwd_win_kernel<DIM, T, MB, STAGE, LOOP, ONE>;
     const size_t lds = ((size_t)GEO_WORDS + (size_t)(wt.cells + (DIM == 3)) * XS) * sizeof(float) + fw.stage_bytes;
     static std::atomic<unsigned long long> lds_raised{0};   // per device, see raise_lds_limit
     if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
@@ -732,21 +735,25 @@ hipError_t launch_k1(const Geo &g, const WinTiles &wt, const FwdWin &fw, const v
     return hipGetLastError();
 }
 
-// the 16-bit loop (when its weight was laid out) and, fp32, the fp32 loop beside it (4.5 us when not selected)
+// fp16 / bf16: the 16-bit loop. fp32: both loops, as kernels of their own where that pays for the launch that is not
+// selected (fw.split, 2D / 3D: see split_loops)
 template <int DIM, typename T, int MB, bool STAGE>
 hipError_t launch_k(const Geo &g, const WinTiles &wt, const FwdWin &fw, const void *xcl, const void *wf,
                     const void *w16, const int *flag, const void *offset, const void *mask, const void *bias, void *y,
                     void *y32, hipStream_t s) {
-    if (w16 != nullptr) {
+    if constexpr (npiece_of<T>() == 2) {
+        if (DIM == 1 || w16 == nullptr || flag == nullptr || !fw.split)
+            return launch_k1<DIM, T, MB, STAGE, LOOP_BOTH, false>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+    }
+    if constexpr (npiece_of<T>() == 1 || DIM > 1) {
         const hipError_t e =
             g.Kn <= wt.tpp
-                ? launch_k1<DIM, T, MB, STAGE, true, true>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s)
-                : launch_k1<DIM, T, MB, STAGE, true, false>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
-        if (e != hipSuccess || npiece_of<T>() == 1 || flag == nullptr) return e;
+                ? launch_k1<DIM, T, MB, STAGE, LOOP_16, true>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s)
+                : launch_k1<DIM, T, MB, STAGE, LOOP_16, false>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
+        if (e != hipSuccess || npiece_of<T>() == 1) return e;
+        if constexpr (npiece_of<T>() == 2)
+            return launch_k1<DIM, T, MB, STAGE, LOOP_F32, false>(g, wt, fw, xcl, wf, w16, flag, offset, mask, bias, y, y32, s);
     }
-    if constexpr (npiece_of<T>() == 2)
-        return launch_k1<DIM, T, MB, STAGE, false, false>(g, wt, fw, xcl, wf, w16, w16 != nullptr ? flag : nullptr, offset,
-                                                          mask, bias, y, y32, s);
     return hipErrorInvalidValue;
 }
 
@@ -795,7 +802,13 @@ size_t x_window_cell_bytes() { return XS * sizeof(float); }
 namespace {
 constexpr double SHARE_US = 8.0, PAIR_US = 2.0, SUM_US = 5.0, SUM_BYTES_PER_US = 4e6;
 constexpr size_t SHARE_BYTES_MAX = (size_t)64 << 20;   // partials of one call
-void split_shares(FwdWin &f, const Geo &g, int mb_max, long long spatial, int slices, int tpp, int npiece, bool lean) {
+// Whether a float32 launch of `us` modelled microseconds runs its two loops as kernels of their own: fewer registers
+// for the launch that is not selected, 4 us. Inference, us a call, one kernel against two: 1D never (512 channels k5 on
+// 16 x 4096 773 / 774, 16 on 100 24 / 27); 2D from 100 (256 channels k3 on 8 x 64x64 222 / 220, 128 on 2 x 100x152
+// 131.4 / 130.0, but 256 on 2 x 64x64 84.7 / 85.3, 16 on 8x8 24 / 27); 3D, whose sampler spills beside a second loop,
+// from 15 (64 channels k3 on 2 x 16x56x56 599 / 542, on 8x20x20 67 / 64, but 16 channels k1 on 4x4x4 28 / 31).
+bool split_loops(int dim, double us) { return dim == 2 ? us >= 100.0 : dim == 3 && us >= 15.0; }
+void split_shares(FwdWin &f, const Geo &g, int dim, int mb_max, long long spatial, int slices, int tpp, int npiece, bool lean) {
     const int npass = (g.Kn + tpp - 1) / tpp, units = npass * slices;
     double best = 0.0;
     for (int mb = mb_max; mb >= 4; mb -= 4) {
@@ -813,6 +826,7 @@ void split_shares(FwdWin &f, const Geo &g, int mb_max, long long spatial, int sl
                 f.mb = mb;
                 f.ksplit = ks;
                 f.units_per = per;
+                f.split = split_loops(dim, us);
             }
         }
     }
@@ -839,7 +853,7 @@ FwdWin plan_fwd_win(const Geo &g, const WinTiles &base, int dim, WinTiles &wt, b
     // 128-row tiles prefetch fewer window cells: not where that costs the window its margin (strided
     // layers, whose samples outside it would go to global memory)
     const bool wide = dim < 3 && g.Mg > 64 && window(8, 0).R[2] >= std::min(window(4, 0).R[2], 4);
-    split_shares(f, g, wide ? 8 : 4, spatial, slices, tpp, base.npiece, lean);
+    split_shares(f, g, dim, wide ? 8 : 4, spatial, slices, tpp, base.npiece, lean);
     const int rows = 16 * f.mb;
     const long long max_cells = (long long)xq_of(f.mb) * NT / 4;
     wt = window(f.mb, 0);

@@ -113,6 +113,7 @@ struct FwdWin {
     int ksplit;          // shares of the (pass, 16-channel slice) units of a tile: 1, or more, each a
                          // workgroup storing its fp32 partial to a plane of y32, summed in order
     int units_per;       // units per share
+    bool split;          // (fp32) the 16-bit and the fp32 loop as two launches
     size_t part_elems;   // floats of the shares' partials (0: one share)
     bool vec;            // 4 consecutive pixels of a tile row are contiguous and 4-aligned in the output
     int Mg_pad, Cg_pad;  // padded weight layout Wf[G][Kn][Mg_pad][Cg_pad]
