@@ -397,9 +397,12 @@ FewPlan plan_few(const Geo &g, int dtype, int dim) {
     // 8 x 65536, 3 / 5 / 7 channels 1591 -> 928, 1542 -> 1506, 1594 -> 2087; 2D k4 on 8 x 128x128, 1 / 2 / 3
     // channels 649 -> 280, 595 -> 548, 655 -> 835; 3D k4 on 2 x 8x28x28, 1 / 2 channels 399 -> 250, 366 -> 486.
     // Small layers have a launch less here: 1D k3 on 4 x 4096, 9 channels 30 -> 22, 2D k4 on 2 x 32x32, 3 / 5
-    // channels 33 -> 28, 33 -> 43.
-    const bool small = (long long)g.NP * g.Kn <= 65536;
-    f.scatter = g.C <= (dim == 1 ? (small ? 9 : 5) : dim == 2 ? (small ? 3 : 2) : 1);
+    // channels 33 -> 28, 33 -> 43. Several offset or mask groups in a conv group take the general kernel's per-lane
+    // path: 1D k3 on 12 x 258, float16, 32 channels in 2 conv and 4 offset groups 56 -> 28.
+    const long long work = (long long)g.NP * g.Kn;
+    const bool small = work <= 65536;
+    f.scatter = g.C <= (dim == 1 ? (small ? 9 : 5) : dim == 2 ? (small ? 3 : 2) : 1) ||
+                (dim == 1 && (g.og > g.G || g.mg > g.G) && work <= 16384);
     const int tiles = (g.NP + BP - 1) / BP;
     // one tile per workgroup up to one per CU, then runs of tiles (each workgroup's partial sums of dW are
     // read back by the reduction)
