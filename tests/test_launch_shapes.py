@@ -122,3 +122,29 @@ def test_float32_forward_loops(record, dim, batch, channels, size, kernel, launc
     than one kernel of both, whose launch that is not selected costs 4 us."""
     r = record(problem(dim, batch, channels, channels, size, [kernel] * dim, padding=kernel // 2))
     assert len(blocks(r["forward"], "fwd_win_kernel")) == launches
+
+
+def test_random_general_problems_take_the_general_kernels(record):
+    import torch
+    from test_gpu_general import SEEDS, general_case
+    codes = {torch.float32: F32, torch.float64: F64, torch.float16: F16, torch.bfloat16: BF16}
+    for seed in SEEDS:
+        dim, transposed, dtype, p = general_case(seed)
+        r = record(problem(dim, p["batch"], p["cin"], p["cout"], p["in_size"], p["kernel"], transposed=transposed,
+                           dtype=codes[dtype], groups=p["groups"], og=p["og"] * p["deformable"], mg=p["mg"] * p["modulated"],
+                           stride=p["stride"], padding=1, bias=p["bias"]))
+        assert r["forward"]["status"] == SUCCESS and r["backward"]["status"] == SUCCESS, (seed, r["backward"]["error"])
+        names = "".join(n for c in r.values() for n, _, _ in c["launches"])
+        for kernel in ("bwd_data_kernel", "bwd_weight_kernel", "fwd_gather_gemm_kernel"):
+            assert kernel in names, (seed, kernel)
+        assert "few_" not in names and "_win_kernel" not in names, seed
+
+
+@pytest.mark.parametrize("batch", [65532, 65533])
+def test_layout_copy_of_many_images(record, batch):
+    """The float32 backward's layout copy has a grid slice per image and one for each job beside it, at most 65535."""
+    r = record(problem(1, batch, 16, 16, [512], [3], padding=1))
+    assert r["backward"]["status"] == SUCCESS
+    (copy,) = [grid for name, grid, _ in r["backward"]["launches"] if "to_cl" in name]
+    assert copy[2] == 65535   # the mask's check, the weight's magnitude, and the bias gradient or one image more
+    assert bool(blocks(r["backward"], "bias_grad_kernel")) == (batch == 65533)

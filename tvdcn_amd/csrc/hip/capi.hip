@@ -767,7 +767,8 @@ tvdcn_status backward_planned(const Plan &pl, const tvdcn_conv_desc *desc, const
         const int bias_c = pl.transposed ? g.C : g.M, bias_s = pl.transposed ? g.Sn : g.Pn;
         const BiasJob bj = {static_cast<const float *>(grad_out), static_cast<float *>(grad_bias), g.B, bias_c, bias_s,
                             accumulate_weight, !pl.transposed};
-        const bool bias_in_copy = dt == kF32 && !cl_in && 2 * copy_blocks(g.C, g.Sn) >= bias_c &&
+        // (and the grid's z holds a slice for it past the images')
+        const bool bias_in_copy = dt == kF32 && !cl_in && 2 * copy_blocks(g.C, g.Sn) >= bias_c && g.B <= 65532 &&
                                   (grad_bias != nullptr || !pl.transposed);
         // (fp32) the 16-bit MFMA operands' largest magnitudes: the weight and X ride on X's layout
         // copy, Z = grad_out on the bias gradient (this block's, accumulated over the blocks),
