@@ -21,7 +21,8 @@ def _desc(p):
         d.in_size[i] = d.kernel[i] = d.stride[i] = d.dilation[i] = 1
     for i in range(p["dim"]):
         d.in_size[i], d.kernel[i] = p["size"][i], p["kernel"][i]
-        d.stride[i], d.padding[i], d.dilation[i] = p["stride"], p["padding"], p["dilation"]
+        d.stride[i] = p["stride"][i] if isinstance(p["stride"], list) else p["stride"]
+        d.padding[i], d.dilation[i] = p["padding"], p["dilation"]
         d.output_padding[i] = p["out_pad"]
     return d
 

@@ -102,7 +102,8 @@ def test_problem_above_2_31_elements():
 def test_forced_batch_blocks_with_unaligned_image_sizes(transposed, dtype, channels_last, images):
     """C = 3 on a 7 x 7 grid: no batch-sized tensor's per-image bytes are a multiple of 16 (float32
     input 588 B), so blocks of 1 or 3 images put later blocks' pointers off 16-byte boundaries (2- or
-    4-byte aligned), which every kernel accepts; blocks of 5 images round down to 4, a multiple of 16
+    4-byte aligned), which the few-channel kernels of these layers accept (the general ones:
+    test_gpu_general.py); blocks of 5 images round down to 4, a multiple of 16
     bytes for every tensor. Batch 7: full blocks and a remainder, against the float64 oracle (float32
     channels-last: the input sampled in place at the block's offset)."""
     case = make_case(2, transposed, batch=7, cin=3, cout=5, kernel=[3, 3], stride=[1, 1], padding=[1, 1],

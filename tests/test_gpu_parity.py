@@ -69,7 +69,7 @@ def check(case, dtype):
         assert e < tb, f"grad_{name} rel err {e}"
 
 
-# flag / group combinations at the reference's test sizes (generic, scalar-channel path)
+# flag / group combinations at the reference's test sizes (few-channel kernels; the general ones: test_gpu_general.py)
 COMBOS = list(itertools.product([1, 2, 3], [False, True], [(True, True), (True, False), (False, True),
                                                               (False, False)]))
 

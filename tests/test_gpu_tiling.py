@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 # data gradient: workgroups (tiles x 16-channel slices x passes of up to nine taps) up to 512 take sixteen
 # waves, more take eight (3D: always sixteen); sixteen waves on 16-bit operands hold a step's fragments of
-# every tap, whatever the number of taps and of 32-channel steps
+# every tap, unless the step's weight is staged in LDS (1D / 2D passes of nine taps)
 DATA_GRADIENT = [
     # dim, batch, cin, cout, size, kernel, transposed
     (1, 128, 64, 16, [5], [3], False),       # 512 workgroups

@@ -108,9 +108,9 @@ def test_deformable_nonfinite_input_fp32(dim):
 
 
 def test_nonfinite_bound_in_a_later_pass_fp32():
-    """25 taps = three passes of the data gradient's window: an inf weight at tap 12 makes only
-    the second pass's bound non-finite, so the window flushes what the first pass accumulated
-    and the second pass scatters through global atomics."""
+    """25 taps = three passes of the data gradient, a workgroup each: an inf weight at tap 12 makes
+    only the second pass's bound non-finite, so it scatters through global atomics beside the
+    windows that the first and the third flush into the same gradient."""
     case = make_case(2, False, batch=2, cin=32, cout=32, kernel=[5, 5], stride=[1, 1], padding=[2, 2],
                      dilation=[1, 1], in_size=[20, 18], out_pad=[0, 0], seed=540)
     case["weight"] = case["weight"].clone()
@@ -130,7 +130,8 @@ def test_nonfinite_bound_in_a_later_pass_fp32():
 
 
 def test_many_taps_multi_pass_fp32():
-    """25 taps: the window accumulates three passes and is rescaled as the bound grows."""
+    """25 taps: three passes, each with a window and a fixed-point scale of its own, flushed into the
+    same gradient by workgroups that may run at once."""
     case = make_case(2, False, batch=2, cin=32, cout=64, kernel=[5, 5], stride=[1, 1], padding=[2, 2],
                      dilation=[1, 1], in_size=[24, 22], out_pad=[0, 0], seed=545, offset_scale=3.0)
     check(case, torch.float32)
