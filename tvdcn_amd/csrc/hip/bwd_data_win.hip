@@ -18,21 +18,23 @@
 // their training step from that alone), and the passes of a small grid run side by side. Sixteen
 // waves of 16 pixels (four per SIMD), or eight of 32 pixels where the K loop counts (see
 // plan_data_win): the 3D epilogue, which waits on LDS and memory, ran 1.63 -> 1.48 ms at 27 taps,
-// 64 channels, 2 x 16x56x56 with sixteen.
+// 64 channels, 2 x 16x56x56 with sixteen. (Each pass flushes a window of its own, which counts where
+// many corners go to global atomics anyway: that 3D layer's training step, by the offsets' standard
+// deviation, 2646 -> 2251 us at half a cell, 2957 -> 2807 at 1.5, but 3426 -> 3520 at 2 and 5210 ->
+// 5397 at 3.)
 //   * K loop over the GEMM-side channels m, operands straight from global memory
 //     into registers (the next step's prefetched while the MFMAs of the current one
-//     run): wave w computes Gt[c][px] for its 32 pixels, so each lane holds four
+//     run): a wave computes Gt[c][px] for its 16 or 32 pixels, so each lane holds four
 //     consecutive channels of one pixel per (tap, 16-pixel block). It runs on
-//     16x16x32 MFMAs, 32 channels per step, from 16-bit operands laid out by
-//     data_prep_kernel (Z and weight splits, one launch): fp16 and bf16 tensors as they are, fp32
-//     tensors as two fp16 pieces each at a per-tensor power-of-two scale, of whose four cross
+//     16x16x32 MFMAs, 32 channels per step, from 16-bit operands laid out in one launch: fp16
+//     and bf16 tensors as they are (prep16.hip), fp32 tensors (data_prep_kernel) as two fp16 pieces each at a per-tensor power-of-two scale, of whose four cross
 //     products the three with i + j <= 1 are summed (the rest are within fp32's own rounding;
 //     3 MFMAs at 16 cycles against 8 fp32 16x16x4 MFMAs at 32 cycles per 32 channels), the
 //     sums scaled back after the K loop. An fp32 operand that is not finite (or at least
 //     0x1.ffp127 in magnitude: a device flag set by the layout kernels) sends the launch down
 //     the fp32 loop (16x16x4 MFMAs, 16 channels per step), which keeps the reference's inf/nan
 //     propagation.
-//   * Epilogue per tap: the geometry of the 256 pixels (one per thread) goes to an
+//   * Epilogue per tap: the geometry of the 256 pixels goes to an
 //     LDS table. The offset/mask gradients are formed in the MFMA layout (4
 //     channels in-lane, two shuffles across the channel quads, one atomic per
 //     pixel and quantity).
@@ -227,7 +229,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     }
 
     // ---- K-loop operands, straight to registers ---------------------------------
-    // B = Z[m][px]: pixel wave * 32 + pb * 16 + lane % 16, m = 4 * (lane / 16) + kk
+    // B = Z[m][px]: pixel wave * PB * 16 + pb * 16 + lane % 16, m = 4 * (lane / 16) + kk
     // A = W[c][m]:  channel c0 + lane % 16, same m; the K order is permuted the same
     //               way on both operands, which leaves the sum unchanged
     int zp[PB];
@@ -496,9 +498,9 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
             }
         };
         // ---- 16-bit K loop with the weight blocks staged in LDS: a step's block (the pass's
-        //      taps x NP pieces, 1 KB each, contiguous in the split layout) is the same for all
-        //      eight waves; read straight from global memory it went eight times through the
-        //      vector memory path. The next step's block is copied global -> LDS (one 1 KB wave
+        //      taps x NP pieces, 1 KB each, contiguous in the split layout) is the same for every
+        //      wave; read straight from global memory it went through the vector memory path once
+        //      for each. The next step's block is copied global -> LDS (one 1 KB wave
         //      instruction per piece, spread over the waves) while this step's MFMAs run, into
         //      the other half of a double buffer; one barrier per step publishes it.
         auto kloop16s = [&]() {
@@ -1145,7 +1147,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         }
         __syncthreads();   // all waves done with the geometry table and the window
 
-        // ---- after the last pass, the window goes out
+        // ---- the pass's window goes out
         if (SCATTER && use_window) flush_window();
     }
 }
