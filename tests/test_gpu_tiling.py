@@ -7,14 +7,15 @@ import torch
 
 import tvdcn
 from helpers import make_case, rel_err
-from test_gpu_parity import check
+from test_gpu_parity import TOL, check, run_gpu, run_oracle
 from test_zz_no_alloc import SCRATCH_BYTES, _desc, _lib, _run
 
 pytestmark = pytest.mark.gpu
 
 
 # data gradient: workgroups (tiles x 16-channel slices x passes of up to nine taps) up to 512 take sixteen
-# waves, more take eight (3D: always sixteen); sixteen waves on 16-bit operands hold a step's fragments of
+# waves, more take eight (3D: always sixteen; the scatter alone with passes in turn: eight float32, sixteen
+# 16-bit); sixteen waves on 16-bit operands hold a step's fragments of
 # every tap, unless the step's weight is staged in LDS (1D / 2D passes of nine taps)
 DATA_GRADIENT = [
     # dim, batch, cin, cout, size, kernel, transposed
@@ -36,6 +37,79 @@ def test_data_gradient_workgroups(case, dtype):
     stride = 2 if transposed else 1
     check(make_case(dim, transposed, batch=batch, cin=cin, cout=cout, kernel=kernel, stride=[stride] * dim,
                     padding=[1] * dim, dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=dim + batch), dtype)
+
+
+# the scatter alone with several passes on grids that fill the chip: the passes in turn in one workgroup, which
+# rescales its window to a pass of larger terms and sends it out before one that is not finite
+PASSES_IN_TURN = [
+    # dim, batch, cin, cout, size, kernel: slices x passes
+    (1, 64, 36, 52, [7], [16]),      # 256 x 2
+    (2, 128, 20, 24, [3, 4], [4, 4]),   # 256 x 2
+    (2, 130, 36, 20, [2, 3], [5, 5]),   # 260 x 3: nine taps, staged weights
+]
+
+
+def passes_case(dim, batch, cin, cout, size, kernel, seed):
+    return make_case(dim, True, batch=batch, cin=cin, cout=cout, kernel=kernel, stride=[1] * dim, padding=[1] * dim,
+                     dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=seed)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", PASSES_IN_TURN, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
+def test_passes_in_turn(case, dtype):
+    check(passes_case(*case, seed=70 + case[0]), dtype)
+
+
+@pytest.mark.parametrize("kind", ["growing", "shrinking", "one_large", "inf_first", "inf_later", "nan_last"])
+@pytest.mark.parametrize("case", PASSES_IN_TURN, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
+def test_passes_in_turn_of_unlike_magnitudes(case, kind):
+    """The mask of each pass on a scale of its own (2^40: nothing of the earlier passes is left in a window on that
+    scale, and nothing of them in the sum's 24 bits), or with a value that is not finite in one of them."""
+    c = passes_case(*case, seed=80 + case[0])
+    kn, dim = c["weight"][0, 0].numel(), case[0]
+    passes = (kn + 8) // 9
+    per = (kn + passes - 1) // passes
+    mask = c["mask"].clone()
+    taps = mask.view(mask.shape[0], kn, -1)
+    for t in range(kn):
+        p = t // per
+        taps[:, t] *= {"growing": 2.0 ** (6 * p), "shrinking": 2.0 ** (-7 * p),
+                       "one_large": 2.0 ** 40 if p == 1 else 1.0}.get(kind, 1.0)
+        if (kind, p) in (("inf_first", 0), ("inf_later", 1)):
+            taps[:, t, 3] = float("inf")
+        if kind == "nan_last" and p == passes - 1:
+            taps[:, t, 3] = float("nan")
+    c["mask"] = mask
+    out, _, _ = run_gpu(c, torch.float32)
+    ref, _ = run_oracle(c, torch.zeros(c["out_shape"], dtype=torch.float64), torch.float32)
+    out = out.detach().double().cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
+    assert torch.isfinite(ref).any() and torch.isfinite(ref).all() == (kind in ("growing", "shrinking", "one_large"))
+    fin = torch.isfinite(ref)
+    e = rel_err(out[fin], ref[fin])
+    assert e < TOL[torch.float32][0], f"forward rel err {e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", PASSES_IN_TURN, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
+def test_passes_in_turn_past_the_range_of_a_cell(case, dtype):
+    """Every (pixel, tap) on the same position with the same term: 2^27 units at most each, of which a cell holds
+    16, so the window wraps in each pass."""
+    c = passes_case(*case, seed=90 + case[0])
+    dim, size, cin = case[0], case[4], case[2]
+    kn, kernel = c["weight"][0, 0].numel(), list(c["weight"].shape[2:])
+    term = 1.9375
+    c["input"], c["mask"] = torch.ones_like(c["input"]), torch.ones_like(c["mask"])
+    c["weight"] = torch.full_like(c["weight"], term / cin)
+    taps = torch.cartesian_prod(*[torch.arange(k) for k in kernel]).view(kn, dim)
+    pixels = torch.cartesian_prod(*[torch.arange(n) for n in size]).view(-1, dim)
+    pos = taps[:, :, None] + pixels.T[None] - 1     # (tap, axis, pixel) at stride 1, padding 1
+    c["offset"] = (2 - pos).to(c["offset"].dtype).expand(c["offset"].shape[0], -1, -1, -1).reshape(c["offset"].shape)
+    out, _, _ = run_gpu(c, dtype)
+    ref, _ = run_oracle(c, torch.zeros(c["out_shape"], dtype=torch.float64), dtype)
+    assert ref.max() > 48 * term
+    e = rel_err(out, ref)
+    assert e < TOL[dtype][0], f"forward rel err {e}"
 
 
 # forward: the (pass, channel slice) units of a tile in one share, in several (whole and ragged last shares,

@@ -124,6 +124,18 @@ def test_float32_forward_loops(record, dim, batch, channels, size, kernel, launc
     assert len(blocks(r["forward"], "fwd_win_kernel")) == launches
 
 
+@pytest.mark.parametrize("dim,batch,cout,size,kernel,in_turn", [
+    (2, 255, 16, [3, 4], 4, True), (2, 128, 32, [3, 4], 4, True), (2, 128, 16, [3, 4], 4, False),   # rounds 2 / 2, 2 / 2, 2 / 1
+    (2, 300, 16, [3, 4], 4, False), (2, 512, 16, [3, 4], 4, True), (2, 512, 16, [3, 4], 3, False),   # 4 / 3, 4 / 4, one pass
+    (1, 256, 16, [20], 16, True), (3, 256, 16, [2, 2, 2], 3, False)])
+def test_passes_of_the_scatter(record, dim, batch, cout, size, kernel, in_turn):
+    """The transposed forward's passes of up to nine taps: in turn in one workgroup where that takes no more rounds of
+    the chip's 256 compute units, a workgroup each otherwise, in 3D and beside the offset gradients."""
+    r = record(problem(dim, batch, 32, cout, size, [kernel] * dim, transposed=True, padding=1))
+    slices, passes = batch * (cout // 16), (kernel ** dim + 8) // 9
+    assert blocks(r["forward"], "bwd_data_win_kernel") == [slices if in_turn else slices * passes]
+
+
 def test_random_general_problems_take_the_general_kernels(record):
     import torch
     from test_gpu_general import SEEDS, general_case

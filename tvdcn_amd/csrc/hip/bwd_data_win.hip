@@ -15,22 +15,23 @@
 // window takes most of the 160 KB of LDS). The passes of a tile are workgroups of their own: a
 // loop over them had the compiler hoist the per-tile values of every phase above it (240-256
 // registers and ~150 spilled scalars per kernel, now 105-176 and 5-60: one-pass layers -2% of
-// their training step from that alone), and the passes of a small grid run side by side. Sixteen
+// their training step from that alone), and the passes of a small grid run side by side. Where a
+// grid of the scatter alone fills the chip without them, the passes take turns in one workgroup
+// (LOOP, an instantiation of its own), which clears and flushes one window (plan_data_win). Sixteen
 // waves of 16 pixels (four per SIMD), or eight of 32 pixels where the K loop counts (see
 // plan_data_win): the 3D epilogue, which waits on LDS and memory, ran 1.63 -> 1.48 ms at 27 taps,
-// 64 channels, 2 x 16x56x56 with sixteen. (Each pass flushes a window of its own, which counts where
-// many corners go to global atomics anyway: that 3D layer's training step, by the offsets' standard
-// deviation, 2646 -> 2251 us at half a cell, 2957 -> 2807 at 1.5, but 3426 -> 3520 at 2 and 5210 ->
-// 5397 at 3.)
+// 64 channels, 2 x 16x56x56 with sixteen. (A window per pass counts where many corners go to global
+// atomics anyway: that 3D layer's training step, by the offsets' standard deviation, 2646 -> 2251 us
+// at half a cell, 2957 -> 2807 at 1.5, but 3426 -> 3520 at 2 and 5210 -> 5397 at 3.)
 //   * K loop over the GEMM-side channels m, operands straight from global memory
 //     into registers (the next step's prefetched while the MFMAs of the current one
 //     run): a wave computes Gt[c][px] for its 16 or 32 pixels, so each lane holds four
 //     consecutive channels of one pixel per (tap, 16-pixel block). It runs on
 //     16x16x32 MFMAs, 32 channels per step, from 16-bit operands laid out in one launch: fp16
-//     and bf16 tensors as they are (prep16.hip), fp32 tensors (data_prep_kernel) as two fp16 pieces each at a per-tensor power-of-two scale, of whose four cross
-//     products the three with i + j <= 1 are summed (the rest are within fp32's own rounding;
-//     3 MFMAs at 16 cycles against 8 fp32 16x16x4 MFMAs at 32 cycles per 32 channels), the
-//     sums scaled back after the K loop. An fp32 operand that is not finite (or at least
+//     and bf16 tensors as they are (prep16.hip), fp32 tensors (data_prep_kernel) as two fp16
+//     pieces each at a per-tensor power-of-two scale, of whose four cross products the three with
+//     i + j <= 1 are summed (the rest are within fp32's own rounding; 3 MFMAs at 16 cycles against
+//     8 fp32 16x16x4 MFMAs at 32 cycles per 32 channels), the sums scaled back after the K loop. An fp32 operand that is not finite (or at least
 //     0x1.ffp127 in magnitude: a device flag set by the layout kernels) sends the launch down
 //     the fp32 loop (16x16x4 MFMAs, 16 channels per step), which keeps the reference's inf/nan
 //     propagation.
@@ -78,9 +79,12 @@ constexpr int FIX_BITS = 29;      // fixed-point headroom: |cell sum| * 2^s_c < 
 // Scatter-only plans (transposed forward; the scatter launch of a split conv backward): the unit
 // follows the largest term the window keeps, |term| * 2^s_c < 2^PREC_BITS, and the cells sum
 // modulo 2^32. An add whose returned old value lies outside [-WRAP_K, WRAP_K) may have wrapped
-// (|add| <= 2^PREC_BITS < 2^31 - WRAP_K); a wrap found there sends the wrapped 2^32 units to
-// global memory, so the held value plus what went out stays the exact integer sum.
-constexpr int PREC_BITS = 26;
+// (|add| <= 2^PREC_BITS <= 2^31 - WRAP_K); a wrap found there sends the wrapped 2^32 units to
+// global memory, so the held value plus what went out stays the exact integer sum. Passes in turn
+// share a unit, which the largest term of them all sets: one bit more (float32, 16 taps on 64 -> 64
+// channels, 8 x 64x64, error against float64: 1.58e-7 with 26 bits, 1.27e-7 with 27; a window
+// and a unit per pass 1.52e-7).
+constexpr int PREC_BITS = 26, PREC_BITS_LOOP = 27;
 constexpr unsigned WRAP_K = 0x78000000u;   // 2^31 - 2^27
 
 // LDS words ahead of the windows: geometry table [WIN_TMAX][BPX] x (position, mask),
@@ -156,7 +160,12 @@ __device__ __forceinline__ unsigned row_sum16(unsigned v) {
     return row_reduce16(v, [](unsigned a, unsigned b) { return a + b; });
 }
 
-template <int DIM, typename T, bool SCATTER, bool COORD, int NW>
+// waves of the passes in turn: the two-piece K loop and the loop's state spill sixteen waves' registers; of 16-bit
+// operands sixteen are faster (16 taps, 64 -> 64, 8 x 64x64: 139 us against 146 with eight)
+template <typename T> constexpr int LOOP_WAVES = npiece_of<T>() == 2 ? 8 : 16;
+
+// LOOP (scatter only): the passes of a tile in turn in one workgroup, which accumulate in one window
+template <int DIM, typename T, bool SCATTER, bool COORD, int NW, bool LOOP>
 __global__ void __launch_bounds__(64 * NW)
 bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wchunks, const uint16_t *zs,
                     const uint16_t *wsplit, const int *flag, const float *__restrict__ xcl,
@@ -169,6 +178,7 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     static_assert(PB >= 1 && NW * PB * 16 == BPX, "one tile of pixels per workgroup");
     // scatter-only: the unit follows the largest kept term, cells sum modulo 2^32 (PREC_BITS)
     constexpr bool PREC = SCATTER && !COORD;
+    static_assert(!LOOP || (PREC && DIM < 3), "passes in turn: the 1D / 2D scatter alone");
 
     extern __shared__ float smem[];
     acc4 *geo = reinterpret_cast<acc4 *>(smem);                // [TMAX][BPX] sampling table (window.h)
@@ -178,6 +188,8 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     float *thr = bsum + NW * BC + BC + 4;                      // [BC] spike thresholds of a pass with spikes
     int *bmax = reinterpret_cast<int *>(thr + BC);             // [BC] largest |G * mask| (float bits, >= 0)
     unsigned *bexp = reinterpret_cast<unsigned *>(bmax + BC);  // [BC] exponent sums + (counts << 20)
+    int *shift = reinterpret_cast<int *>(bsum);                // [BC] (LOOP) rescale of what the window holds, in the
+                                                               // words of the first wave's bounds, which are read
     // (xg: the offset / mask gradients read X from global memory; no X window)
     const bool xg = COORD && wt.xglobal != 0;
     float *xwin = smem + fixed_words(NW);                          // [cells][XS] X window (COORD)
@@ -197,8 +209,8 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     const int ct = L % wt.c_tiles;
     L /= wt.c_tiles;
     const int npass = (g.Kn + wt.tpp - 1) / wt.tpp;
-    const int t0 = L % npass * wt.tpp;
-    L /= npass;
+    const int t_first = LOOP ? 0 : L % npass * wt.tpp;
+    if (!LOOP) L /= npass;
     const int n_sp = g.B * wt.ntile[0] * wt.ntile[1] * wt.ntile[2];
     Tile tile;
     tile.init(g, wt, L % n_sp, ct, L / n_sp);
@@ -272,8 +284,8 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
     //      per channel (gx_nchw)
     // thread = (channel tid % 16, cells tid / 16, + STEP, ...) or, gx_nchw, (channel tid / STEP,
     // cells tid % STEP, + STEP, ...); FB cells' values are read before any is used (one LDS
-    // latency per batch)
-    auto flush_window = [&]() {
+    // latency per batch). keep: the window is used again (cleared as read, barrier at the end)
+    auto flush_window = [&](bool keep) {
         constexpr int FB = 8;
         constexpr int STEP = NT / 16;
         static_assert(NT / STEP == BC, "both thread maps step STEP cells per channel");
@@ -314,12 +326,15 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
 #pragma unroll
             for (int j = 0; j < FB; ++j) {
                 if (iv[j] == 0) continue;
+                if (keep) iwin[c * cst + cell0 + j * STEP] = 0;
                 if (si[j] >= 0) atomic_add(gbase + (size_t)si[j] * gps, ldexpf((float)iv[j], -se));
             }
         }
+        if (keep) __syncthreads();
     };
 
-    {
+    bool win_data = false;   // (LOOP) the window holds an earlier pass's values
+    for (int t0 = t_first;; t0 += wt.tpp) {   // (without LOOP: once, and no loop to the compiler)
         const int ntaps = min(wt.tpp, g.Kn - t0);
 
         // ---- sampling table of the pass, one (tap, pixel) per thread ------------------
@@ -674,12 +689,22 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
             };
             // PREC: the scale of the pass from the largest term the window keeps (kmax; a pass
             // with spikes keeps the terms up to their threshold); bc (the sum of every term) only
-            // tells whether the pass is finite
+            // tells whether the pass is finite. LOOP: coarsened to what the window holds; a pass
+            // that is not finite leaves that scale to the flush.
             auto set_scale_prec = [&](float kmax, float bc) {
                 const unsigned long long bad = __ballot(!isfinite(bc));
                 int e = 0;
                 if (kmax > 0.f && isfinite(kmax)) frexpf(kmax, &e);   // kmax < 2^e
-                scl[tid] = PREC_BITS - e;
+                int sc = (LOOP ? PREC_BITS_LOOP : PREC_BITS) - e;
+                if constexpr (LOOP) {
+                    const int held = win_data ? scl[tid] : sc;
+                    if (bad != 0ull) sc = held;
+                    sc = min(sc, held);
+                    shift[tid] = held - sc;
+                    bmax[tid] = 0;   // for the next pass
+                    bexp[tid] = 0u;
+                }
+                scl[tid] = sc;
                 if (tid == 0) scl[BC] = bad != 0ull;
             };
             const float no_lim[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
@@ -735,6 +760,23 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
             // not finite (or 3D spikes): the pass goes to global float atomics (inf / nan propagate
             // as in the reference)
             if (no_window) spikes = false;
+            if constexpr (LOOP) {
+                if (win_data && no_window) {
+                    flush_window(true);
+                    win_data = false;
+                } else if (win_data) {
+                    // rescale to nearest (halves up); a shift of 31 or more leaves at most a unit
+                    const int c = tid / (NT / BC), sh = shift[c];
+                    if (sh > 0) {
+                        for (int cell = tid % (NT / BC); cell < cst; cell += NT / BC) {
+                            const int v = iwin[c * cst + cell];
+                            iwin[c * cst + cell] = sh >= 31 ? 0 : (v >> sh) + ((v >> (sh - 1)) & 1);
+                        }
+                    }
+                    __syncthreads();
+                }
+                win_data = win_data || (wt.cells > 0 && !no_window);
+            }
             use_window = wt.cells > 0 && !no_window;
 #pragma unroll
             for (int v = 0; v < 4; ++v) sexp[v] = scl[mq + v];
@@ -1147,8 +1189,14 @@ bwd_data_win_kernel(const Geo g, const WinTiles wt, const T *z, const float *wch
         }
         __syncthreads();   // all waves done with the geometry table and the window
 
-        // ---- the pass's window goes out
-        if (SCATTER && use_window) flush_window();
+        // ---- the window goes out (LOOP: with the last pass)
+        if constexpr (LOOP) {
+            if (t0 + wt.tpp < g.Kn) continue;
+            if (win_data) flush_window(false);
+        } else {
+            if (SCATTER && use_window) flush_window(false);
+        }
+        break;
     }
 }
 
@@ -1212,16 +1260,17 @@ template <bool SCATTER, bool COORD> size_t lds_bytes(const WinTiles &t) {
            (size_t)t.wstage;
 }
 
-template <int DIM, typename T, bool SCATTER, bool COORD, int NW>
+template <int DIM, typename T, bool SCATTER, bool COORD, int NW, bool LOOP = false>
 hipError_t launch_w(const Geo &g, const WinTiles &tl, const void *z, const void *wchunks, const void *zs,
                     const void *wsplit, const int *flag, const void *xcl, const void *offset, const void *mask,
                     void *gx_cl, void *goff, void *gmask, hipStream_t s, bool gx_nchw) {
-    auto kern = bwd_data_win_kernel<DIM, T, SCATTER, COORD, NW>;
+    auto kern = bwd_data_win_kernel<DIM, T, SCATTER, COORD, NW, LOOP>;
     const size_t lds = lds_bytes<SCATTER, COORD>(tl);
     static std::atomic<unsigned long long> lds_raised{0};   // per device, see raise_lds_limit
     if (const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kern), lds_raised); e != hipSuccess)
         return e;
-    const long long blocks = (long long)g.G * g.B * tl.ntile[0] * tl.ntile[1] * tl.ntile[2] * tl.c_tiles * ((g.Kn + tl.tpp - 1) / tl.tpp);
+    const long long blocks = (long long)g.G * g.B * tl.ntile[0] * tl.ntile[1] * tl.ntile[2] * tl.c_tiles *
+                             (LOOP ? 1 : (g.Kn + tl.tpp - 1) / tl.tpp);
     if (blocks == 0) return hipErrorInvalidValue;
     return launch_block_runs(blocks, 64 * NW, [&](int first, unsigned n) {
         hipLaunchKernelGGL(kern, dim3(n), dim3(64 * NW), lds, s, g, tl, static_cast<const T *>(z),
@@ -1236,6 +1285,10 @@ template <int DIM, typename T, bool SCATTER, bool COORD>
 hipError_t launch_k(const Geo &g, const WinTiles &tl, const void *z, const void *wchunks, const void *zs,
                     const void *wsplit, const int *flag, const void *xcl, const void *offset, const void *mask,
                     void *gx_cl, void *goff, void *gmask, hipStream_t s, bool gx_nchw) {
+    if constexpr (SCATTER && !COORD && DIM < 3)
+        if (tl.loop)
+            return launch_w<DIM, T, SCATTER, COORD, LOOP_WAVES<T>, true>(g, tl, z, wchunks, zs, wsplit, flag, xcl, offset,
+                                                                        mask, gx_cl, goff, gmask, s, gx_nchw);
     if (tl.waves == 16)
         return launch_w<DIM, T, SCATTER, COORD, 16>(g, tl, z, wchunks, zs, wsplit, flag, xcl, offset, mask, gx_cl, goff,
                                                     gmask, s, gx_nchw);
@@ -1405,8 +1458,15 @@ WinTiles plan_data_win(const Geo &g, int dtype, int dim, bool scatter, bool coor
     // eight waves share each weight fragment's read between two pixel blocks, which the K loop of a
     // large grid needs; sixteen hide more latency, which bounds grids of up to two rounds of the
     // chip (one workgroup per CU) and the 3D epilogue
-    const long long blocks = (long long)g.G * g.B * t.ntile[0] * t.ntile[1] * t.ntile[2] * t.c_tiles * npass;
+    const long long slices = (long long)g.G * g.B * t.ntile[0] * t.ntile[1] * t.ntile[2] * t.c_tiles, blocks = slices * npass;
     t.waves = dim == 3 || blocks <= 512 ? 16 : 8;
+    // The scatter alone, several passes: in turn in one workgroup, with one window to clear and to flush,
+    // unless the passes as workgroups of their own end in fewer rounds of the chip (one workgroup per CU).
+    // 16 taps at stride 2, float32 / float16, apart -> in turn: 256 -> 128 channels, 8 x 32x32, 132 -> 113 us /
+    // 103 -> 93; 64 -> 64, 8 x 64x64, 183 -> 164 / 168 -> 139; 1D, 128 -> 128, 8 x 1024, 84 -> 75 / 64 -> 60.
+    // Apart on 128 workgroups in turn (256 -> 128, 2 x 32x32: 67 us against 97).
+    t.loop = dim < 3 && scatter && !coord && npass > 1 && (slices + 255) / 256 * npass <= (blocks + 255) / 256;
+    if (t.loop) t.waves = dtype == kF32 ? LOOP_WAVES<float> : LOOP_WAVES<__half>;
     // per window cell: the fixed-point accumulators (scatter) and / or the X values
     // (offset/mask gradients), as the launches this plan serves need them
     // (+ BC * 16 words: the fixed-point window's stride rounding)

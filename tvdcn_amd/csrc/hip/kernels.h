@@ -73,6 +73,7 @@ struct WinTiles {
     int c_tiles, m_steps;
     int tpp;             // taps per pass (<= WIN_TMAX)
     int waves;           // waves per data-gradient workgroup: 8 (32 pixels each) or 16 (16 pixels each)
+    bool loop;           // (scatter only) the passes of a tile in turn in one workgroup
     size_t chunk_elems;  // floats of the re-laid-out weight
     // 16-bit MFMA operands of the data gradient (16x16x32 MFMAs over 32 GEMM-side channels per
     // step): fp32 tensors split into two fp16 pieces each (per-tensor power-of-two scale), fp16 /
