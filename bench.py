@@ -296,8 +296,8 @@ SUITE = [(2, torch.float32), (3, torch.float32), (4, torch.float32), (5, torch.f
          (5, torch.bfloat16)]
 
 
-TRAFFIC_KERNELS = {"gather_gemm": "fwd_win_kernel<2, float, 8, true, true, true>",
-                   "data_grad": "bwd_data_win_kernel<2, float, true, true, 8>",
+TRAFFIC_KERNELS = {"gather_gemm": "fwd_win_kernel<2, float, 8, true, 1, true>",
+                   "data_grad": "bwd_data_win_kernel<2, float, true, true, 8, false>",
                    "weight_grad": "bwd_weight_win_kernel<2, float, true, 2, 1, 9, 32, true>"}
 
 

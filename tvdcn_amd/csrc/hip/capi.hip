@@ -212,6 +212,7 @@ tvdcn_status make_plan(const tvdcn_conv_desc *d, Plan &pl, int64_t batch, bool l
     pl.ww = plan_weight_win(g, pl.wn_w, pl.dim);
     pl.fw = plan_fwd_win(g, pl.wn_s, pl.dim, pl.wn_f, lean);
     pl.few = plan_few(g, pl.dtype, pl.dim);
+    // windowed plans come first (their layers of 4, 8 or 12 channels were not timed on the few-channel kernels)
     if (pl.wn_s.ok) pl.few.ok = pl.few.scatter = false;
     const bool cl_in = (d->flags & TVDCN_FLAG_CHANNELS_LAST) != 0;
     // (1D only: there a window row is the tile's 256 pixels + margins, whole lines of each channel;

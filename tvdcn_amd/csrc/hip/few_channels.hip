@@ -380,15 +380,17 @@ size_t data_lds(const Geo &g, int dtype, bool weight) {
 
 FewPlan plan_few(const Geo &g, int dtype, int dim) {
     FewPlan f{};
-    // Columns of up to 128 values, or 200 on grids of up to a tile per CU, and weights of up to 24576: beyond either the general kernels'
-    // wider tiles win (float32, us a training step, general -> here: 3 -> 64 k3 on 8 x 224x224 5476 ->
+    // Columns of up to 128 values, or 200 on grids of up to a tile per CU, and weights of up to 24576: beyond
+    // either the general kernels' wider tiles win (float32, us a training step, general -> here: 3 -> 64 k3 on 8 x 224x224 5476 ->
     // 1535, 5 -> 512 k3 on 4 x 64x64 652 -> 280, 10 -> 512 666 -> 679, 14 -> 512 668 -> 882, 21 -> 30 on
     // 20x20 459 -> 214, 30 -> 30 on 16 x 128x128 4406 -> 9081). A fused mask
-    // activation's gradient is finished in the accumulation type, which 16-bit gradients here never are.
+    // activation's gradient is finished in the accumulation type, which 16-bit gradients here never are (the
+    // forward of such a layer follows its backward; not timed apart).
     // Fewer than 2^30 pixels: four threads each stay below HIP's 2^32 of a launch, and a run of tiles that
     // ends past the last pixel below 2^31.
     const long long column = (long long)g.C * g.Kn;
-    f.ok = g.NP < 1 << 30 && (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) && (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype, true) <= WIN_LDS_TARGET &&
+    f.ok = g.NP < 1 << 30 && (column <= 128 || (column <= 200 && g.NP <= 256 * BP)) &&
+           (long long)g.M * g.Cg * g.Kn <= 24576 && data_lds(g, dtype, true) <= WIN_LDS_TARGET &&
            (g.mask_act == 0 || dtype == kF32 || dtype == kF64);
     if (!f.ok || g.NP == 0) return f;
     // The scatter alone (the transposed forward): a lane per pixel, so that an atomic instruction reaches up to 64
