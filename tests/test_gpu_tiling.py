@@ -60,6 +60,16 @@ def test_passes_in_turn(case, dtype):
     check(passes_case(*case, seed=70 + case[0]), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("kw", [dict(deformable=False, modulated=False, stride=[1, 1], in_size=[5, 4]),
+                                dict(stride=[3, 3], in_size=[10, 25])], ids=["offset_free", "scatter_apart"])
+def test_passes_in_turn_of_a_backward(kw, dtype):
+    """The input gradient of a convolution by itself: nothing but it to compute from the columns, or a window too small
+    beside the one of the offset gradients. 128 images of two slices, two passes."""
+    check(make_case(2, False, batch=128, cin=20, cout=24, kernel=[4, 4], padding=[1, 1], dilation=[1, 1],
+                    out_pad=[0, 0], seed=77, **kw), dtype)
+
+
 @pytest.mark.parametrize("kind", ["growing", "shrinking", "one_large", "inf_first", "inf_later", "nan_last"])
 @pytest.mark.parametrize("case", PASSES_IN_TURN, ids=lambda c: "-".join(str(v) for v in c).replace(" ", ""))
 def test_passes_in_turn_of_unlike_magnitudes(case, kind):

@@ -136,6 +136,15 @@ def test_passes_of_the_scatter(record, dim, batch, cout, size, kernel, in_turn):
     assert blocks(r["forward"], "bwd_data_win_kernel") == [slices if in_turn else slices * passes]
 
 
+@pytest.mark.parametrize("kw,launches", [
+    (dict(batch=128, size=[5, 4], og=0, mg=0), [256]), (dict(batch=128, size=[10, 25], stride=3), [256, 512]),
+    (dict(batch=32, size=[20, 20]), [512])])
+def test_passes_of_a_backward(record, kw, launches):
+    """The input gradient without offset / mask gradients, with theirs in a launch of their own, in one with theirs."""
+    r = record(problem(2, cin=20, cout=24, kernel=[4, 4], padding=1, **kw))
+    assert blocks(r["backward"], "bwd_data_win_kernel") == launches
+
+
 def test_random_general_problems_take_the_general_kernels(record):
     import torch
     from test_gpu_general import SEEDS, general_case
