@@ -151,6 +151,48 @@ def test_forward_shares(case, dtype):
                     seed=40 + dim + batch), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case", [FORWARD[3] + (1,), PASSES_IN_TURN[1] + (True, 1), PASSES_IN_TURN[2] + (True, 1)],
+                         ids=["shares", "two_passes", "three_passes"])
+def test_captured_graph(case, dtype):
+    """A forward and backward of several shares, and of passes in turn, captured on a stream of its own and replayed on
+    rewritten inputs with eager calls on the default stream in between: each replay gives the eager result. Float
+    atomics add the same terms in another order; bfloat16 outputs then round to neighbours (2^-8) now and then."""
+    dim, batch, cin, cout, size, kernel, transposed, padding = case
+    c = make_case(dim, transposed, batch=batch, cin=cin, cout=cout, kernel=kernel, stride=[1] * dim,
+                  padding=[padding] * dim, dilation=[1] * dim, out_pad=[0] * dim, in_size=size, seed=95)
+    op = tvdcn.deform_conv_transpose2d if transposed else tvdcn.deform_conv2d
+    names = ("input", "weight", "offset", "mask", "bias")
+    ts = [c[n].to("cuda:0", dtype).requires_grad_(True) for n in names]
+    gy = torch.rand(c["out_shape"], device="cuda:0").to(dtype)
+
+    def run():
+        y = op(*ts, stride=1, padding=padding)
+        return (y,) + torch.autograd.grad(y, ts, gy)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            run()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        outs = run()
+    g = torch.Generator(device="cuda:0").manual_seed(96)
+    for rep in range(3):
+        with torch.no_grad():
+            for t in ts:
+                t.copy_(torch.randn(t.shape, device="cuda:0", generator=g))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, r in zip(("output",) + names, outs, run()):
+            e = rel_err(a.detach(), r.detach())
+            assert e < (1e-5 if dtype == torch.float32 else 2.0 ** -8), f"replay {rep}: {name} {e}"
+
+
 def test_forward_without_room_for_partial_sums():
     """The allocation-free forward takes a problem whose shares' partials alone exceed its scratch array: in
     one share, the same sum in another order. Its 4608 positive terms reach a float32 accumulator in at least
